@@ -35,6 +35,7 @@ SOURCES = [
     "permutation.cpp",
     "wire.cpp",
     "contraction_kernels.hip",
+    "gemm_split_kernels.hip",
     "contraction_noalloc.hip",
     "contraction_f16_kernels.hip",
     "permutation_kernels.hip",

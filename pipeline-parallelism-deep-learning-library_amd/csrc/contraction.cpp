@@ -415,6 +415,23 @@ int load_mode_half(uintptr_t base, uint64_t off, uint64_t sb, uint64_t srow, uin
     return LOAD_S;
 }
 
+// Whether a tiled plan runs on the bf16 matrix cores with every element in three pieces
+// (gemm_split.h): the tiles of 128x128 and more, K chunks long enough to fill its pipeline, at least the four
+// rows and columns a thread loads at once, and operand tiles whose elements lie within 32 bits of
+// bytes of their first one, which is how the kernel addresses them.
+bool pieces_fit(const GemmArgs& t) {
+    if (t.kernel != KERN_TILE && t.kernel != KERN_DIRECT && t.kernel != KERN_PIPE) return false;
+    if (t.tile < GEMM_BM || t.tile_n < GEMM_BN || t.kgroups != 1) return false;
+    const uint32_t last = t.k - (t.splits - 1) * t.k_chunk;
+    if (std::min(t.k_chunk, last) < PIECES_MIN_K || t.m < 4 || t.n < 4) return false;
+    auto near = [](uint64_t rows, int64_t srow, int64_t sk) {
+        const uint64_t limit = 1ull << 29;  // elements, half of 2^32 bytes
+        const uint64_t r = static_cast<uint64_t>(srow), k = static_cast<uint64_t>(sk);
+        return r < limit / 512 && k < limit / 64 && rows * r + 16 * k < limit;
+    };
+    return near(t.tile, t.a_sm, t.a_sk) && near(t.tile_n, t.b_sn, t.b_sk);
+}
+
 // The f16 plans: the same kinds, on the f16 kernels. No split-K: one f64 tile per output block.
 void plan_half(const View& a, const View& b, const View& c, const Merged& mg, float alpha,
                float beta, bool reads_inputs, Plan& p) {
@@ -998,6 +1015,9 @@ Plan plan_merged(const View& a, const View& b, const View& c, const Merged& mg, 
             info.tile_m = info.tile_n = GEMM_BM;
         }
     }
+    t.splits = splits;
+    t.k_chunk = chunk;
+    t.pieces = pieces_fit(t) ? 1 : 0;
     info.kgroups = t.kgroups;
     info.kernel = t.kernel == KERN_SK       ? LG_KERNEL_STREAMK
                   : t.kernel == KERN_TILE   ? LG_KERNEL_TILE
@@ -1005,8 +1025,6 @@ Plan plan_merged(const View& a, const View& b, const View& c, const Merged& mg, 
                   : t.kernel == KERN_DIRECT ? LG_KERNEL_DIRECT
                   : t.kernel == KERN_SMALL  ? LG_KERNEL_SMALL
                                             : LG_KERNEL_WAVE;
-    t.splits = splits;
-    t.k_chunk = chunk;
     info.splits = splits;
     info.k_chunk = chunk;
     info.workgroups = gemm_workgroups(t);

@@ -470,6 +470,12 @@ void launch_gemm(Context* ctx, hipStream_t s, const GemmArgs& args, int a_mode, 
          {"gemm_f32_pl<MN,K>", "gemm_f32_pl<MN,MN>", "gemm_f32_pl<MN,S>"},
          {"gemm_f32_pl<S,K>", "gemm_f32_pl<S,MN>", "gemm_f32_pl<S,S>"}}};
     if (args.kernel > KERN_SK) fail_invalid("unknown GEMM kernel");
+    if (args.pieces != 0) {
+        const char* piece_name = launch_gemm_pieces(s, args, groups);
+        check_launch("gemm launch");
+        note_launch(ctx, piece_name);
+        return;
+    }
     static const char* const deep[3][3] = {
         {"gemm_f32_pl32<K,K>", "gemm_f32_pl32<K,MN>", "gemm_f32_pl32<K,S>"},
         {"gemm_f32_pl32<MN,K>", "gemm_f32_pl32<MN,MN>", "gemm_f32_pl32<MN,S>"},

@@ -1,0 +1,488 @@
+// The fp32 GEMM on the bf16 matrix cores: every operand element as three bf16 pieces.
+//
+// An f32 has 24 significant bits and a bf16 has 8, so x = x0 + x1 + x2 with x0 = bf16(x),
+// x1 = bf16(x - x0), x2 = x - x0 - x1, each step exact: the three pieces hold the f32 whole. A
+// product is then six bf16 products, a0b0 + (a0b1 + a1b0) + (a1b1 + a0b2 + a2b0); the three left
+// out are below 2^-26 of it. bf16 products are exact in f32 and one
+// v_mfma_f32_32x32x16_bf16 adds sixteen of them into an f32 accumulator, so a sum over K is
+// rounded about 6 K / 16 times instead of the K times of v_mfma_f32_32x32x2_f32.
+//
+// The pieces cover f32's range down to 2^-110 or so, below which the last of them would need
+// bits that bf16 does not have, and up to bf16's largest value. A workgroup that meets a smaller
+// element, or whose sums come out as anything but finite numbers (an infinity or a NaN in an
+// operand or an overflow: x - x0 turns them into NaN), computes its tile again with the f32
+// matrix instruction on the operands themselves (b3_redo).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "gemm_dlds.h"
+
+namespace lg {
+namespace gemm_detail {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned short ushortx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
+// Four floats that are only known to be 4-byte aligned (global_load_dwordx4 needs no more).
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int B3_BK = 16;  // K depth of one slice
+
+// LDS image of one operand's slice, R rows: three planes (one per piece), each of two chunks (k 0-7 and
+// 8-15), each of four classes (row % 4), each of R / 4 rows of 16 bytes (eight bf16). A
+// thread converts a block of four rows by four k: for each row of the block the wave writes 16
+// neighbouring rows of one class, 8 bytes each. A fragment read takes 32 rows by 16 bytes:
+// eight consecutive lanes are two neighbours in each of four classes, which the classes' 32-byte padding
+// puts on distinct banks; the chunk's 64-byte padding does so for the two chunks of a write.
+template <int R>
+struct B3Geo {
+    static constexpr int CLS = R * 4 + 64;
+    static constexpr int CH = 4 * CLS + 64;
+    static constexpr int PL = 2 * CH;
+    static constexpr int BYTES = 3 * PL;
+};
+
+// Elements below 2^(B3_LEAST - 127) and not zero go to b3_redo. (From exponent 17 on all three
+// pieces of an f32 are exact; checked on every exponent and 2^21 elements each.)
+constexpr uint32_t B3_LEAST = 24;
+
+// (x, y) -> three packed pairs of bf16 pieces. `low` keeps the least 2 |x0| - 1 (mod 2^16) seen,
+// in which zero counts as the largest. Thirteen VALU instructions a pair, four cycles each, and up to six of
+// them hide behind every MFMA. (v_dot2_f32_bf16 would do the subtraction and the unpacking in one, exactly,
+// but it does not run beside an MFMA: two of them cost an MFMA's time and a half.)
+struct B3Low {
+    ushortx2 v = {0xffff, 0xffff};
+    uint32_t two = 0x00020002u, ones = 0xffffffffu;
+    __device__ __forceinline__ B3Low() {
+        __asm__("" : "+s"(two));
+        __asm__("" : "+v"(ones));
+    }
+    __device__ __forceinline__ void see(uint32_t q) {
+        uint32_t d;
+        __asm__("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(d) : "v"(q), "s"(two), "v"(ones));
+        v = __builtin_elementwise_min(v, __builtin_bit_cast(ushortx2, d));
+    }
+    __device__ __forceinline__ bool tiny() const {
+        return min(static_cast<uint32_t>(v[0]), static_cast<uint32_t>(v[1])) < 2u * (B3_LEAST << 7) - 1u;
+    }
+};
+__device__ __forceinline__ void b3_split(float x, float y, uint32_t (&q)[3], B3Low& low) {
+    q[0] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
+    low.see(q[0]);
+    x = x - __builtin_bit_cast(float, q[0] << 16);
+    y = y - __builtin_bit_cast(float, q[0] & 0xffff0000u);
+    q[1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
+    x = x - __builtin_bit_cast(float, q[1] << 16);
+    y = y - __builtin_bit_cast(float, q[1] & 0xffff0000u);
+    q[2] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
+}
+
+// One thread's 4 x 4 block of an operand slice (rows 4 rq .. 4 rq + 3, k 4 k4 .. 4 k4 + 3), in the order in
+// which it is loaded: LOAD_K and LOAD_S v[row][k], LOAD_MN v[k][row].
+struct B3Block {
+    floatx4 v[4];
+};
+
+// Where a thread's block lies: byte offsets from the tile's first element of the slice, uniform strides,
+// and the LDS byte address of each of its rows (EDGE: rows past the operand's end are
+// the last ones again, and rows before the tile's first are not written).
+template <int MODE, int R, bool EDGE>
+struct B3Loader {
+    using G = B3Geo<R>;
+    const float* base;  // the operand at the tile's first row (EDGE, LOAD_MN: see init) and current k
+    int64_t srow, sk;
+    uint32_t off[4];   // byte offset of load i (one offset and uniform strides unless EDGE)
+    uint32_t lds[4];   // byte address of row i in plane 0 (EDGE: 0xffffffff = not written)
+    uint32_t k4;
+
+    // p: the operand at (row 0 of the batch plane, first k). m0: the tile's first row, rows: the
+    // operand's row count, t: the thread's number among the R threads that load this operand.
+    __device__ __forceinline__ void init(const float* p, int64_t srow_, int64_t sk_, uint32_t m0,
+                                         uint32_t rows, uint32_t t) {
+        srow = srow_;
+        sk = sk_;
+        k4 = t & 3u;
+        const uint32_t rq = t >> 2;
+        const uint32_t at = (k4 >> 1) * G::CH + (k4 & 1u) * 8u;
+        uint32_t row0 = m0 + 4 * rq;  // first row of the block
+        uint32_t first = m0;          // row that `base` points at
+        if constexpr (EDGE && MODE == LOAD_MN) {
+            // A block that would cross the end starts four rows before it.
+            row0 = min(row0, rows - 4);
+            first = min(m0, rows - 4);
+        }
+        base = p + static_cast<int64_t>(first) * srow;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t row = EDGE && MODE != LOAD_MN ? min(row0 + i, rows - 1) : row0 + i;
+            if constexpr (MODE == LOAD_MN) {
+                off[i] = (row0 - first) * 4u;
+            } else if constexpr (EDGE) {
+                off[i] = static_cast<uint32_t>((row - first) * srow) * 4u;
+            } else {
+                off[i] = static_cast<uint32_t>((row0 - first) * srow) * 4u;
+            }
+            if constexpr (MODE != LOAD_MN) off[i] += k4 * 4u * static_cast<uint32_t>(sk) * 4u;
+            else off[i] += k4 * 4u * static_cast<uint32_t>(sk) * 4u;
+            const uint32_t r = EDGE && MODE == LOAD_MN ? row0 + i - m0 : 4 * rq + i;
+            lds[i] = static_cast<int32_t>(r) < 0 ? 0xffffffffu : at + (r & 3u) * G::CLS + (r >> 2) * 16u;
+        }
+    }
+    __device__ __forceinline__ const float* at(int i) const {
+        // Load i's uniform part: row i of the block (LOAD_K, LOAD_S) or its k i (LOAD_MN).
+        const float* b = base;
+        if constexpr (MODE == LOAD_MN) b += i * sk;
+        else if constexpr (!EDGE) b += i * srow;
+        return b;
+    }
+    __device__ __forceinline__ void load(B3Block& x) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (MODE == LOAD_S) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    x.v[i][j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(at(i) + j * sk) + off[i]);
+                }
+            } else {
+                x.v[i] = *reinterpret_cast<const floatx4u*>(reinterpret_cast<const char*>(at(i)) + off[i]);
+            }
+        }
+    }
+    // The last slice's `left` < 16 k: zero past them.
+    __device__ __forceinline__ void load_tail(B3Block& x, uint32_t left) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (MODE == LOAD_MN) {
+                x.v[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (4 * k4 + i < left) {
+                    x.v[i] = *reinterpret_cast<const floatx4u*>(reinterpret_cast<const char*>(at(i)) + off[i]);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    x.v[i][j] = 0.0f;
+                    if (4 * k4 + j < left) {
+                        x.v[i][j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(at(i) + j * sk) + off[i]);
+                    }
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void advance() { base += B3_BK * sk; }
+
+    // Row i of the block: its pieces into a stage.
+    template <bool SCALE>
+    __device__ __forceinline__ void store_row(char* stage, const B3Block& x, int i, float scale, B3Low& low) const {
+        float e[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            e[j] = MODE == LOAD_MN ? x.v[j][i] : x.v[i][j];
+            if constexpr (SCALE) e[j] = scale * e[j];
+        }
+        uint32_t lo[3], hi[3];
+        b3_split(e[0], e[1], lo, low);
+        b3_split(e[2], e[3], hi, low);
+        if (!(EDGE && MODE == LOAD_MN) || lds[i] != 0xffffffffu) {
+            char* q = EDGE && MODE == LOAD_MN ? stage + lds[i] : stage + lds[0] + i * G::CLS;
+#pragma unroll
+            for (int s = 0; s < 3; ++s) *reinterpret_cast<uintx2*>(q + s * G::PL) = uintx2{lo[s], hi[s]};
+        }
+    }
+};
+
+// The tile's sums in plain f32 (v_mfma_f32_32x32x2_f32), straight from memory: for tiles whose elements
+// the bf16 pieces do not cover. Slow and rare.
+template <int FM, int FN, int WN>
+__device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const float* B, uint32_t m0,
+                                                  uint32_t n0, uint32_t klen, int wave, int lane,
+                                                  floatx16 (&acc)[FM][FN]);
+
+template <int FM, int FN>
+__device__ __forceinline__ void b3_zero(floatx16 (&acc)[FM][FN]) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+}
+
+// One row of blocks: the six products of A block `a` with each B block, small ones first, each B piece
+// for the last time as early as the order allows (piece 2 in the first product, piece 1 by the third).
+template <int FN, typename F>
+__device__ __forceinline__ void b3_block(const bf16x8 (&a)[3], const bf16x8 (&b)[FN][3], floatx16 (&acc)[FN], F&& after) {
+    constexpr int ta[6] = {0, 1, 0, 2, 1, 0}, tb[6] = {2, 1, 1, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ta[t]], b[j][tb[t]], acc[j], 0, 0, 0);
+        after(t);
+    }
+}
+
+// One (32 FM WM) x (32 FN WN) tile over k [0, klen) from A and B (batch plane, first k): acc. Returns
+// whether some element was too small for its pieces.
+template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
+__device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const float* A, const float* B,
+                                        uint32_t m0, uint32_t n0, uint32_t klen, floatx16 (&acc)[FM][FN]) {
+    constexpr int RA = 32 * FM * WM, RB = 32 * FN * WN;
+    using GA = B3Geo<RA>;
+    using GB = B3Geo<RB>;
+    constexpr int ST = GA::BYTES + GB::BYTES;
+    constexpr int WA = RA / 64, WB = RB / 64;  // waves that load A, then B
+    constexpr int NX = FM == 4 ? 2 : 4, EARLY = FM == 4 ? 0 : 2;
+    static_assert(WA + WB <= WM * WN, "one block of a slice per thread");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    // This lane's fragment addresses (row lane % 32 of a block, chunk lane / 32).
+    const uint32_t fr = (lane & 3) * 1u, fq = ((lane & 31) >> 2) * 16u, fh = lane >> 5;
+    const uint32_t fa = fr * GA::CLS + fq + fh * GA::CH + wm * FM * 128;
+    const uint32_t fb = fr * GB::CLS + fq + fh * GB::CH + wn * FN * 128 + GA::BYTES;
+    const uint32_t full = klen / B3_BK, left = klen - full * B3_BK;
+    B3Low low;
+
+    auto loop = [&](auto* loader, auto scaled, float scale, char* mine) __attribute__((always_inline)) {
+        using LD = std::remove_pointer_t<decltype(loader)>;
+        constexpr bool LOADS = !std::is_same_v<LD, void*>;
+        constexpr bool SCALE = decltype(scaled)::value;
+        // Slice s passes through the registers x[s % NX] into stage s % 2. Step s multiplies slice s. All
+        // of stage s % 2 is read and all of slice s + 1 written when the last row of blocks
+        // begins: the step's one barrier stands there, and behind it, among that row's MFMAs, the
+        // first fragments of slice s + 1 are read and the first EARLY rows of slice s + 2
+        // converted into the stage just read; the other rows are converted in step s + 1 before its
+        // barrier, which ends with the loads of slice s + 2 + NX into the same registers. Past the last slice the
+        // last one is loaded again.
+        const uint32_t slices = full + (left != 0);
+        B3Block x[NX];
+        auto fetch = [&](uint32_t s, B3Block& to) __attribute__((always_inline)) {
+            if constexpr (LOADS) {
+                if (s != 0 && s < slices) loader->advance();
+                if (EDGE && left != 0 && s + 1 >= slices) loader->load_tail(to, left);
+                else loader->load(to);
+            }
+        };
+        auto put_row = [&](int i, int stage, const B3Block& from) __attribute__((always_inline)) {
+            if constexpr (LOADS) loader->template store_row<SCALE>(mine + stage * ST, from, i, scale, low);
+        };
+        bf16x8 a[2][3], b[FN][3];
+        auto read_a = [&](bf16x8 (&to)[3], int i, int stage) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) to[q] = *reinterpret_cast<const bf16x8*>(smem + fa + stage * ST + q * GA::PL + i * 128);
+        };
+        auto read_b = [&](int q, int stage) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j) b[j][q] = *reinterpret_cast<const bf16x8*>(smem + fb + stage * ST + q * GB::PL + j * 128);
+        };
+        auto step = [&](auto phase, uint32_t s) __attribute__((always_inline)) {
+            constexpr int U = decltype(phase)::value, P = U & 1, X1 = (U + 1) % NX, X2 = (U + 2) % NX;
+            constexpr int MG = 6 * FN;
+            // VALU instructions after each MFMA: a row takes 26, and the loop's own a few more.
+            constexpr int V = LOADS ? ((4 - EARLY) * 28 + (FM - 1) * MG - 1) / ((FM - 1) * MG) : 0;
+            constexpr int VL = LOADS ? (EARLY * 28 + MG - 1) / MG : 0;
+#pragma unroll
+            for (int i = 0; i + 1 < FM; ++i) {
+                read_a(a[(i + 1) & 1], i + 1, P);
+                // This row of blocks' share of the conversion.
+#pragma unroll
+                for (int r = EARLY + i * (4 - EARLY) / (FM - 1); r < EARLY + (i + 1) * (4 - EARLY) / (FM - 1); ++r) {
+                    put_row(r, P ^ 1, x[X1]);
+                }
+                b3_block<FN>(a[i & 1], b, acc[i], [](int) {});
+                // One read after each of the first MFMAs, the conversion's VALU work and writes spread over all.
+#pragma unroll
+                for (int q = 0; q < MG; ++q) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (q < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    if constexpr (V > 0) {
+                        __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+                        if (q % 3 == 2) __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            wait_lgkm0();
+            __builtin_amdgcn_s_barrier();
+            constexpr int L = (FM - 1) & 1;
+#pragma unroll
+            for (int r = 0; r < EARLY; ++r) put_row(r, P, x[X2]);
+            b3_block<FN>(a[L], b, acc[FM - 1], [&](int t) {
+                if (t == 0) read_b(2, P ^ 1);
+                if (t == 2) {
+                    read_b(1, P ^ 1);
+                    read_a(a[L ^ 1], 0, P ^ 1);
+                }
+                if (t == 5) read_b(0, P ^ 1);
+            });
+            if constexpr (VL > 0) {
+#pragma unroll
+                for (int q = 0; q < MG; ++q) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (q > 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, VL, 0);
+                    if (q % 3 == 2) __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
+                }
+            }
+            if constexpr (L == 0) {
+#pragma unroll
+                for (int q = 0; q < 3; ++q) a[0][q] = a[1][q];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(s + 1 + NX, x[X1]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int s = 0; s < NX; ++s) fetch(s, x[s]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) put_row(r, 0, x[0]);
+#pragma unroll
+        for (int r = 0; r < EARLY; ++r) put_row(r, 1, x[1]);
+        fetch(NX, x[0]);
+        wait_lgkm0();
+        __builtin_amdgcn_s_barrier();
+        read_a(a[0], 0, 0);
+        read_b(2, 0);
+        read_b(1, 0);
+        read_b(0, 0);
+        uint32_t s = 0;
+        if constexpr (NX == 4) {
+            for (; s + 3 < slices; s += 4) {
+                step(std::integral_constant<int, 0>{}, s);
+                step(std::integral_constant<int, 1>{}, s + 1);
+                step(std::integral_constant<int, 2>{}, s + 2);
+                step(std::integral_constant<int, 3>{}, s + 3);
+            }
+            if (s < slices) step(std::integral_constant<int, 0>{}, s);
+            if (s + 1 < slices) step(std::integral_constant<int, 1>{}, s + 1);
+            if (s + 2 < slices) step(std::integral_constant<int, 2>{}, s + 2);
+        } else {
+            for (; s + 1 < slices; s += 2) {
+                step(std::integral_constant<int, 0>{}, s);
+                step(std::integral_constant<int, 1>{}, s + 1);
+            }
+            if (s < slices) step(std::integral_constant<int, 0>{}, s);
+        }
+    };
+    auto with = [&](auto* loader, float scale, char* mine) __attribute__((always_inline)) {
+        if (scale != 1.0f) loop(loader, std::true_type{}, scale, mine);
+        else loop(loader, std::false_type{}, scale, mine);
+    };
+    if (wave < WA) {
+        B3Loader<AM, RA, EDGE> ld;
+        ld.init(A, p.a_sm, p.a_sk, m0, p.m, tid);
+        with(&ld, p.scale_b ? 1.0f : p.alpha, smem);
+    } else if (wave < WA + WB) {
+        B3Loader<BMD, RB, EDGE> ld;
+        ld.init(B, p.b_sn, p.b_sk, n0, p.n, tid - RA);
+        with(&ld, p.scale_b ? p.alpha : 1.0f, smem + GA::BYTES);
+    } else {
+        void* none = nullptr;
+        loop(&none, std::false_type{}, 1.0f, smem);
+    }
+    return low.tiny();
+}
+
+template <int FM, int FN, int WN>
+__device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const float* B, uint32_t m0,
+                                                  uint32_t n0, uint32_t klen, int wave, int lane,
+                                                  floatx16 (&acc)[FM][FN]) {
+    const int wm = wave / WN, wn = wave % WN;
+    const uint32_t lr = lane & 31, h = lane >> 5;
+    const float alpha_a = p.scale_b ? 1.0f : p.alpha, alpha_b = p.scale_b ? p.alpha : 1.0f;
+    const float *ar[FM], *br[FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) ar[i] = A + static_cast<int64_t>(min(m0 + (wm * FM + i) * 32 + lr, p.m - 1)) * p.a_sm;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) br[j] = B + static_cast<int64_t>(min(n0 + (wn * FN + j) * 32 + lr, p.n - 1)) * p.b_sn;
+    b3_zero(acc);
+    for (uint32_t k = 0; k < klen; k += 2) {
+        const uint32_t kk = k + h;
+        float a[FM], b[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) a[i] = kk < klen ? alpha_a * ar[i][kk * p.a_sk] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) b[j] = kk < klen ? alpha_b * br[j][kk * p.b_sk] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+}
+
+// gemm_f32_b3<AM, BMD, WM, WN, FM, FN, EDGE>: C = beta * C + sum_k (alpha * a) * b, or raw split-K partials,
+// on (32 FM WM) x (32 FN WN) tiles of WM x WN waves: 256x256 and 256x128 and 128x256 tiles with eight waves
+// (the first with 4 x 2 blocks each, so that a piece read from LDS feeds twice the products), 128x128 with
+// four. EDGE: ragged tiles or a K that is no multiple of 16. Operands pass through registers, where
+// they are split, so a load needs no alignment beyond its elements' and edges cost no second path.
+//
+// Bound: the chip's power. 1748 TFLOP/s of bf16 MFMA is what it sustains with nothing else running (1.74 of
+// 2.4 GHz), 291 TFLOP/s of this product; the 256x256 tiles keep the matrix cores 78 % busy at 1.70 GHz, the
+// rest of the power going into fragment reads and conversions. Fewer stalls alone do not help: the same
+// kernel without a schedule was busy 69 % at 1.87 GHz and 3 % slower. Against v_mfma_f32_32x32x2_f32 on the same
+// tiles: 4096^3 931 -> 570-580 us (148 -> 237 TFLOP/s), 32 x 1024^3 483 -> 310 us (142 -> 222), a layer's three
+// products and elementwise work at 2048 x 2048 x 8192 1554 -> 1108 us. Error against f64 on
+// normal operands: 1.0e-6 (4096^3), 4.9e-7 (K = 1024), before 1.1e-6 and 5.7e-7.
+template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
+__global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b3(GemmArgs p) {
+    constexpr int RA = 32 * FM * WM, RB = 32 * FN * WN;
+    constexpr int ST = B3Geo<RA>::BYTES + B3Geo<RB>::BYTES;
+    __shared__ __attribute__((aligned(16))) char smem[2 * ST];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t plane, tm, tn;
+    decode_tile<RA == 256 ? 4 : 8>(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, &plane, &tm, &tn);
+    const uint32_t bi = plane / p.splits, split = plane - bi * p.splits;
+    const uint32_t m0 = tm * RA, n0 = tn * RB, kb = split * p.k_chunk;
+    const uint32_t klen = min(p.k - kb, p.k_chunk);
+    const float* A = p.a + static_cast<int64_t>(bi) * p.a_sb + static_cast<int64_t>(kb) * p.a_sk;
+    const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
+    floatx16 acc[FM][FN];
+    b3_zero(acc);
+    bool bad = b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, acc);
+    // x * 0 is 0 unless x is infinite or NaN. Rows and columns past the output's edge hold
+    // whatever the stages held, and do not count.
+    const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
+    float z = 0.0f;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float t = acc[i][j][r] * 0.0f;
+                if (!EDGE || (m0 + (wm * FM + i) * 32 + (r >> 2) * 8 + h * 4 + (r & 3) < p.m &&
+                              n0 + (wn * FN + j) * 32 + lr < p.n)) {
+                    z = z + t;
+                }
+            }
+    if (__syncthreads_or(bad || z != 0.0f)) b3_redo<FM, FN, WN>(p, A, B, m0, n0, klen, wave, lane, acc);
+
+    float* C = p.partial != nullptr ? p.partial + static_cast<int64_t>(plane) * p.m * p.n
+                                    : p.c + static_cast<int64_t>(bi) * p.c_sb;
+    const int64_t c_sm = p.partial != nullptr ? static_cast<int64_t>(p.n) : p.c_sm;
+    const int64_t c_sn = p.partial != nullptr ? 1 : p.c_sn;
+    const float beta = p.partial != nullptr ? 0.0f : p.beta;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const uint32_t col = n0 + (wn * FN + j) * 32 + lr;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t row = m0 + (wm * FM + i) * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+                if (EDGE && (row >= p.m || col >= p.n)) continue;
+                float* q = C + row * c_sm + col * c_sn;
+                float v = acc[i][j][r];
+                if (beta != 0.0f) v = beta * *q + v;
+                *q = v;
+            }
+        }
+}
+
+}  // namespace gemm_detail
+}  // namespace lg

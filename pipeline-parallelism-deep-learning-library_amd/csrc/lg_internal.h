@@ -190,7 +190,14 @@ struct GemmArgs {
     // KERN_PIPE: K depth of one LDS slice, 16 or 32.
     uint32_t slice_k;
     uint32_t* counters;  // KERN_SK: one ticket counter per range boundary, zero between launches
+    // 1: the same tiles and splits on the bf16 matrix cores, every element as three bf16 pieces
+    // (gemm_f32_b3, gemm_split.h), chosen by the planner's pieces_fit.
+    uint32_t pieces;
 };
+// K chunks below this stay on the f32 matrix instruction.
+constexpr uint32_t PIECES_MIN_K = 64;
+// Launches the three-piece kernel for args.pieces; returns the name for the launch log.
+const char* launch_gemm_pieces(hipStream_t s, const GemmArgs& args, uint32_t groups);
 
 // Dot products (M = N = 1): C[b] = beta*C[b] + sum_k (alpha*a[b][k])*b[b][k]. Split along K
 // into `splits` workgroups per product writing partial sums, which a second launch adds in

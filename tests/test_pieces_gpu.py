@@ -1,0 +1,116 @@
+"""The f32 GEMM on three bf16 pieces per element (gemm_f32_b3), at the edges of its tiles, slices and range.
+
+Every product is compared with the exact one in f64 under the bound of an f32 dot product,
+(K + 2) u sum |a||b| plus C's own rounding.
+"""
+import numpy as np
+import pytest
+
+from linalg_hip import contraction as C
+from helpers import Layout, Tensor, rng
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+
+def _product(ctx, pool, a, b, ta, tb, alpha=1.0, beta=0.0, c0=None, stride=1):
+    """alpha * a @ b + beta * c0 through the library; `ta` / `tb` store an operand column-major,
+    `stride` 2 leaves no unit stride in A."""
+    m, k = a.shape
+    n = b.shape[1]
+    la = Layout.transposed(m, k) if ta else Layout.dense([m, k])
+    stored = (a.T if ta else a).ravel()
+    if stride == 2:
+        la = Layout(0, [m, k], [2, 2 * m] if ta else [2 * k, 2])
+        stored = np.repeat(stored, 2)[:-1]
+    lb = Layout.transposed(k, n) if tb else Layout.dense([k, n])
+    A = Tensor(pool, la, np.ascontiguousarray(stored))
+    B = Tensor(pool, lb, np.ascontiguousarray((b.T if tb else b).ravel()))
+    c = np.full((m, n), np.nan, np.float32) if c0 is None else c0.astype(np.float32)
+    Cc = Tensor(pool, Layout.dense([m, n]), c.ravel().copy())
+    C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
+    name = [x for x in ctx.launches() if x.startswith("gemm")][-1]
+    return Cc.read()[: m * n].reshape(m, n).copy(), name
+
+
+def _check(got, a, b, alpha, beta, c0):
+    k = a.shape[1]
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want = alpha * (a64 @ b64)
+    bound = (k + 2) * U * abs(alpha) * (np.abs(a64) @ np.abs(b64)) + 1e-44
+    if beta:
+        want = want + beta * c0
+        bound = bound + 2 * U * np.abs(beta * c0) + U * np.abs(want)
+    assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
+
+
+@pytest.mark.parametrize("m,n,k,ta,tb,stride", [
+    (2045, 1930, 77, False, False, 1),    # odd rows and pitches: 4-byte aligned 128-bit loads, K tail of 13
+    (2045, 1929, 64, True, True, 1),      # A along M, B along K, the shortest K, one ragged column
+    (1921, 2048, 65, True, False, 1),     # one row past a tile, K tail of 1
+    (2048, 1923, 79, False, True, 1),     # three columns past a tile, K tail of 15
+    (1924, 1924, 96, True, False, 1),     # whole quads past a tile
+    (2048, 2048, 80, False, False, 1),    # full tiles, five slices
+    (2048, 2048, 90, True, True, 2),      # no unit stride in A
+    (1921, 1925, 67, False, False, 2),
+])
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (-0.3, 0.75)])
+def test_tile_edges(ctx, pool, m, n, k, ta, tb, stride, alpha, beta):
+    g = rng(9100 + m + n + k)
+    a = g.standard_normal((m, k)).astype(np.float32)
+    b = g.standard_normal((k, n)).astype(np.float32)
+    c0 = g.standard_normal((m, n)).astype(np.float32) if beta else None
+    alpha = float(np.float32(alpha))
+    got, name = _product(ctx, pool, a, b, ta, tb, alpha, beta, c0, stride)
+    assert name.startswith("gemm_f32_b3"), name
+    _check(got, a, b, alpha, beta, c0)
+
+
+def test_pieces_hold_the_element_whole(ctx, pool):
+    """A times a permutation matrix is A's columns, bit for bit, over f32's range down to 2^-100."""
+    n = 2048
+    g = rng(9200)
+    a = np.ldexp(g.uniform(1, 2, (n, n)), g.integers(-100, 100, (n, n))).astype(np.float32)
+    a *= g.choice([-1, 1], (n, n)).astype(np.float32)
+    perm = g.permutation(n)
+    b = np.zeros((n, n), np.float32)
+    b[perm, np.arange(n)] = 1.0
+    got, name = _product(ctx, pool, a, b, False, False)
+    assert name.startswith("gemm_f32_b3"), name
+    assert np.array_equal(got, a[:, perm])
+
+
+@pytest.mark.parametrize("what", ["inf", "nan", "huge", "tiny", "subnormal", "zero"])
+def test_elements_outside_the_pieces(ctx, pool, what):
+    """Infinities, NaNs, elements past bf16's largest and below what three pieces hold: the
+    products of f32 arithmetic, wherever in K and in the tile they stand."""
+    m, n, k = 2045, 1930, 77
+    g = rng(9300)
+    a = g.standard_normal((m, k)).astype(np.float32)
+    b = g.standard_normal((k, n)).astype(np.float32)
+    if what in ("inf", "nan"):
+        v = np.float32(np.inf if what == "inf" else np.nan)
+        a[5, 76], a[700, 0], a[2044, 30], b[40, 1929] = v, -v, v, v
+    elif what == "huge":
+        a[5, 76] = a[2044, 3] = np.finfo(np.float32).max
+        b *= np.float32(2.0 ** -10)
+    elif what == "tiny":
+        a *= np.float32(2.0 ** -115)
+        b *= np.float32(2.0 ** 60)
+    elif what == "subnormal":
+        a[700] = (g.integers(1, 1 << 20, k) * 2.0 ** -149).astype(np.float32)
+        b *= np.float32(2.0 ** 100)
+        a[:700] = 0
+        a[701:] = 0
+    else:
+        a[:] = 0
+    got, name = _product(ctx, pool, a, b, False, False)
+    assert name.startswith("gemm_f32_b3"), name
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        fine = np.isfinite(want)
+        assert np.array_equal(np.isnan(want), np.isnan(got))
+        assert np.array_equal(want[~fine & ~np.isnan(want)], got[~fine & ~np.isnan(want)])
+        bound = (k + 2) * U * (np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64)))
+    assert np.all(np.abs(got[fine] - want[fine]) <= bound[fine] + 1e-44)
