@@ -24,6 +24,8 @@
 // add +0 (turning a -0 sum into +0) or 0 * inf.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "lg_internal.h"
 
 namespace lg {
@@ -211,6 +213,255 @@ __global__ __launch_bounds__(QT) void gemm16_seq(Gemm16SeqArgs p) {
     }
 }
 
+// gemm16_chain<HK, NB, AV, BV>: the same chain on the f32 matrix cores. v_mfma_f32_16x16x4_f32
+// adds its four products to an output one after another in k order, each as one fused
+// multiply-add with f32 subnormals kept (checked bit for bit against fmaf over 400 random
+// tiles, subnormal sums among them). A fused multiply-add rounds as the chain's multiply and add do
+// wherever the product itself needs no rounding, and that is the rule here: f16 elements have 11
+// significant bits and bf16 ones 8, so (alpha * a) * b has at most 24 when alpha has at most 2 or 8
+// (1, -0.5, 0.75, ...; the host's chain_fuses), and f16 products cannot leave f32's range. bf16
+// ones can, so a tile that meets an |alpha * a| or |b| outside [2^-55, 2^62) that is not zero is computed
+// again with separate multiplies and adds (`odd`).
+// A last slice that is not full is padded with products (-0) * 1: adding -0 changes no sum.
+//
+// 32 NB x 32 NB outputs per 256-thread workgroup, four waves in 2 x 2 of NB x NB blocks of 16x16. All
+// threads load: each 16 k of one row, so a slice is 2048 / (32 NB) deep. Stages hold f32,
+// [16 k][k % 4][row][k / 4], so a lane's four steps are one 128-bit read, lanes on distinct banks. Two stages, the
+// loads of a slice one slice ahead of its conversion, in registers. Bound: the f32 matrix rate, 157 TFLOP/s. 2048 x 4096 x
+// 1024 against the VALU kernel gemm16_seq: bf16 411 -> 164 us, f16 411 -> 159 us; 128 x 1408 x 1024, a few
+// workgroups whose chains alone set the time, 146 -> 15 us on 32x32 tiles.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <bool VEC>
+struct Raw16 {
+    u32x4 v[2];
+};
+template <>
+struct Raw16<false> {
+    uint16_t v[16];
+};
+
+template <int HK, int NB, bool AV, bool BV>
+__global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
+    constexpr int R = 32 * NB, BK = 2048 / R, KG = BK / 16;
+    constexpr int OP = R * BK;  // floats of one operand's stage
+    __shared__ __attribute__((aligned(16))) float stage[2][2 * OP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1, lr = lane & 15, lk = lane >> 4;
+    // Tiles in groups of eight rows, each XCD (workgroups go round the eight in turn) a run of them.
+    const uint32_t total = gridDim.x, xcd = blockIdx.x & 7u, q8 = total >> 3, r8 = total & 7u;
+    const uint32_t lin = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (blockIdx.x >> 3);
+    const uint32_t group = lin / (8 * p.tiles_n), gm = min(p.tiles_m - group * 8, 8u), in = lin - group * 8 * p.tiles_n;
+    const uint32_t m0 = (group * 8 + in % gm) * R, n0 = (in / gm) * R;
+    bool odd = false;  // an element whose products may round was met
+
+    f32x4 acc[NB][NB];
+    // Output (i, j, r) of this lane, and the chain's start.
+    auto row_of = [&](int i, int r) { return m0 + (wm * NB + i) * 16 + lk * 4 + r; };
+    auto col_of = [&](int j) { return n0 + (wn * NB + j) * 16 + lr; };
+    auto start = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    acc[i][j][r] = 0.0f;
+                    if (p.beta != 0.0f && row_of(i, r) < p.m && col_of(j) < p.n) {
+                        acc[i][j][r] = p.beta * widen<HK>(p.c[static_cast<int64_t>(row_of(i, r)) * p.c_sm + col_of(j)]);
+                    }
+                }
+    };
+    start();
+    const uint32_t slices = (p.k + BK - 1) / BK;
+    auto loop = [&](auto vec, const uint16_t* src, int64_t s_row, int64_t s_k, uint32_t rows, float scale,
+                    float pad, float* to) __attribute__((always_inline)) {
+        constexpr bool VEC = decltype(vec)::value;
+        // This thread's row of the tile and 16-k group of the slice: consecutive lanes along the
+        // operand's contiguous axis. Rows past the end repeat the last one. Addresses are the slice's
+        // (uniform) first element and a 32-bit offset of the lane's.
+        const uint32_t t = tid & 127;
+        const uint32_t row = s_k == 1 ? t / KG : t % R, kg = s_k == 1 ? t % KG : t / R;
+        const uint32_t off = static_cast<uint32_t>(min(row, rows - 1) * s_row + kg * 16 * s_k) * 2u;
+        float* mine = to + kg * 16 * R + row * 4;
+        Raw16<VEC> x;
+        auto load = [&](uint32_t s) __attribute__((always_inline)) {
+            const char* base = reinterpret_cast<const char*>(src + static_cast<int64_t>(s) * BK * s_k);
+            if ((s + 1) * BK <= p.k) {
+                if constexpr (VEC) {
+                    x.v[0] = *reinterpret_cast<const u32x4*>(base + off);
+                    x.v[1] = *reinterpret_cast<const u32x4*>(base + 16 + off);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) x.v[j] = *reinterpret_cast<const uint16_t*>(base + j * s_k * 2 + off);
+                }
+            } else {
+                const uint32_t k = s * BK + kg * 16;
+                if constexpr (VEC) {
+                    // Whole runs of eight: K is a multiple of eight here.
+                    x.v[0] = x.v[1] = u32x4{0, 0, 0, 0};
+                    if (k < p.k) x.v[0] = *reinterpret_cast<const u32x4*>(base + off);
+                    if (k + 8 < p.k) x.v[1] = *reinterpret_cast<const u32x4*>(base + 16 + off);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) {
+                        x.v[j] = 0;
+                        if (k + j < p.k) x.v[j] = *reinterpret_cast<const uint16_t*>(base + j * s_k * 2 + off);
+                    }
+                }
+            }
+        };
+        auto put = [&](uint32_t s) __attribute__((always_inline)) {
+            const uint32_t k = s * BK + kg * 16;
+            float f[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                uint16_t h;
+                if constexpr (VEC) h = static_cast<uint16_t>(x.v[j >> 3][(j >> 1) & 3] >> (16 * (j & 1)));
+                else h = x.v[j];
+                f[j] = scale * widen<HK>(h);
+            }
+            if constexpr (HK == 1) {
+                uint32_t low = 0xffffffffu, high = 0;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const uint32_t u = __builtin_bit_cast(uint32_t, f[j]) << 1;
+                    low = min(low, u - 1);  // zero: the largest
+                    high = max(high, u);
+                }
+                odd = odd || low < ((127u - 55u) << 24) - 1 || high >= ((127u + 62u) << 24);
+            }
+            if (k + 16 > p.k) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (k + j >= p.k) f[j] = pad;
+            }
+            float* q = mine + (s & 1) * 2 * OP;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(q + c * 4 * R) = f32x4{f[c], f[4 + c], f[8 + c], f[12 + c]};
+        };
+        auto multiply = [&](uint32_t s) __attribute__((always_inline)) {
+            const float* as = stage[s & 1] + lk * 4 * R + (wm * NB * 16 + lr) * 4;
+            const float* bs = stage[s & 1] + OP + lk * 4 * R + (wn * NB * 16 + lr) * 4;
+#pragma unroll
+            for (int g = 0; g < KG; ++g) {
+                f32x4 a[NB], b[NB];
+#pragma unroll
+                for (int i = 0; i < NB; ++i) a[i] = *reinterpret_cast<const f32x4*>(as + g * 16 * R + i * 64);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) b[j] = *reinterpret_cast<const f32x4*>(bs + g * 16 * R + j * 64);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < NB; ++i)
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+            }
+        };
+        load(0);
+        put(0);
+        if (slices > 1) load(1);
+        __syncthreads();
+        for (uint32_t s = 0; s < slices; ++s) {
+            if (s + 1 < slices) put(s + 1);
+            if (s + 2 < slices) load(s + 2);
+            multiply(s);
+            __syncthreads();
+        }
+    };
+    if (wave < 2) {
+        loop(std::integral_constant<bool, AV>{}, p.a + static_cast<int64_t>(m0) * p.a_sm, p.a_sm, p.a_sk, p.m - m0,
+             p.alpha, -0.0f, stage[0]);
+    } else {
+        loop(std::integral_constant<bool, BV>{}, p.b + static_cast<int64_t>(n0) * p.b_sn, p.b_sn, p.b_sk, p.n - n0,
+             1.0f, 1.0f, stage[0] + OP);
+    }
+
+    if (HK == 1 && __syncthreads_or(odd)) {
+        // Slow and rare: the chain as written, every element from memory.
+        start();
+        const uint16_t *ar[NB * 4], *br[NB];
+#pragma unroll
+        for (int i = 0; i < NB * 4; ++i) ar[i] = p.a + static_cast<int64_t>(min(row_of(i >> 2, i & 3), p.m - 1)) * p.a_sm;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) br[j] = p.b + static_cast<int64_t>(min(col_of(j), p.n - 1)) * p.b_sn;
+        for (uint32_t k = 0; k < p.k; ++k) {
+            float bv[NB];
+#pragma unroll
+            for (int j = 0; j < NB; ++j) bv[j] = widen<HK>(br[j][k * p.b_sk]);
+#pragma unroll
+            for (int i = 0; i < NB * 4; ++i) {
+                const float av = p.alpha * widen<HK>(ar[i][k * p.a_sk]);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    const float prod = av * bv[j];
+                    acc[i >> 2][j][i & 3] = acc[i >> 2][j][i & 3] + prod;
+                }
+            }
+        }
+    }
+
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (row_of(i, r) < p.m && col_of(j) < p.n) {
+                    p.c[static_cast<int64_t>(row_of(i, r)) * p.c_sm + col_of(j)] = narrow<HK>(acc[i][j][r]);
+                }
+            }
+}
+
+// Whether (alpha * a) * b never needs rounding (see gemm16_chain): alpha has at most 2 (f16) or 8 (bf16)
+// significant bits and a moderate exponent.
+bool chain_fuses(uint32_t kind, float alpha) {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, alpha);
+    const int e = static_cast<int>((bits >> 23) & 0xffu) - 127;
+    const uint32_t below = kind == 1 ? 0xffffu : 0x3fffffu;  // mantissa bits past the first 8, past the first 2
+    return e >= -10 && e <= 30 && (bits & below) == 0;
+}
+
+template <int HK, int NB>
+void launch_chain_nb(hipStream_t s, const Gemm16SeqArgs& a, uint32_t groups) {
+    // 128-bit loads: rows contiguous along K, 16-byte aligned, K in whole runs of eight.
+    auto vec = [&](const uint16_t* q, int64_t s_row, int64_t s_k) {
+        return s_k == 1 && s_row % 8 == 0 && a.k % 8 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0;
+    };
+    const bool av = vec(a.a, a.a_sm, a.a_sk), bv = vec(a.b, a.b_sn, a.b_sk);
+    const dim3 grid(groups);
+    if (av && bv) hipLaunchKernelGGL((gemm16_chain<HK, NB, true, true>), grid, dim3(256), 0, s, a);
+    else if (av) hipLaunchKernelGGL((gemm16_chain<HK, NB, true, false>), grid, dim3(256), 0, s, a);
+    else if (bv) hipLaunchKernelGGL((gemm16_chain<HK, NB, false, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((gemm16_chain<HK, NB, false, false>), grid, dim3(256), 0, s, a);
+}
+
+// The kernel's 32-bit offsets within a tile's slice.
+bool chain_near(const Gemm16SeqArgs& a) {
+    auto near = [](int64_t s_row, int64_t s_k) {
+        const uint64_t r = static_cast<uint64_t>(s_row), k = static_cast<uint64_t>(s_k);
+        return r < (1u << 22) && k < (1u << 22);
+    };
+    return near(a.a_sm, a.a_sk) && near(a.b_sn, a.b_sk);
+}
+
+template <int HK>
+void launch_chain(hipStream_t s, Gemm16SeqArgs a) {
+    // The largest tiles whose grid still gives every compute unit two workgroups; the
+    // smallest ones for anything less.
+    uint32_t tile = 128;
+    while (tile > 32 && gemm16_seq_workgroups(a.m, a.n, tile) < 2 * GEMM16_SEQ_CUS) tile /= 2;
+    a.tile = tile;
+    a.tiles_m = (a.m + tile - 1) / tile;
+    a.tiles_n = (a.n + tile - 1) / tile;
+    const uint64_t groups = gemm16_seq_workgroups(a.m, a.n, tile);
+    if (groups == 0 || groups * 256 > 0xffffffffull) fail_invalid("16-bit gemm grid exceeds one launch");
+    const uint32_t g = static_cast<uint32_t>(groups);
+    if (tile == 128) launch_chain_nb<HK, 4>(s, a, g);
+    else if (tile == 64) launch_chain_nb<HK, 2>(s, a, g);
+    else launch_chain_nb<HK, 1>(s, a, g);
+}
+
 }  // namespace
 
 uint64_t gemm16_seq_workgroups(uint32_t m, uint32_t n, uint32_t tile) {
@@ -224,7 +475,10 @@ void launch_gemm16_seq(Context* ctx, hipStream_t s, const Gemm16SeqArgs& args) {
         fail_invalid("16-bit gemm grid does not match its extents");
     }
     const dim3 grid(static_cast<uint32_t>(groups));
-    if (args.kind == 1) {
+    if (args.k > 0 && chain_fuses(args.kind, args.alpha) && chain_near(args)) {
+        if (args.kind == 1) launch_chain<1>(s, args);
+        else launch_chain<0>(s, args);
+    } else if (args.kind == 1) {
         if (args.tile == 64) {
             hipLaunchKernelGGL((gemm16_seq<1, 4>), grid, dim3(QT), 0, s, args);
         } else {

@@ -1,0 +1,59 @@
+"""The 16-bit Backend gemm on the f32 matrix cores (gemm16_chain): CpuBackend's bits at the
+edges of its tiles and slices and of the range in which its products need no rounding."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import rng
+from test_backend_gpu import run16, same16, hb  # noqa: F401  (hb: the backend fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(kind, x):
+    x = np.ascontiguousarray(x, dtype=np.float32)
+    return oracle.f32_to_f16(x) if kind == "f16" else oracle.f32_to_bf16(x)
+
+
+def _check(hb, kind, layout, a, b, c, m, k, n, alpha, beta):
+    a16, b16, c16 = _bits(kind, a.ravel()), _bits(kind, b.ravel()), _bits(kind, c.ravel())
+    got = run16(hb, kind, layout, a16, b16, c16, m, k, n, alpha, beta)
+    want = oracle.gemm_seq_16(kind, alpha, beta, a16.reshape(m, k), b16.reshape(k, n), c16.reshape(m, n))
+    assert same16(kind, got, want)
+
+
+# 128x128 tiles (529 of them, ragged), 64x64 (552) and 32x32, with K around their slices of 16, 32
+# and 64; K in whole runs of eight takes 128-bit loads.
+@pytest.mark.parametrize("m,k,n", [(2900, 16, 2820), (2817, 17, 2944), (2823, 40, 2900), (1500, 32, 1450),
+                                   (1409, 33, 1473), (1481, 104, 1472), (70, 64, 45), (33, 65, 97),
+                                   (31, 1, 32), (64, 136, 64), (1, 191, 700)])
+@pytest.mark.parametrize("kind,layout", [("f16", "at"), ("f16", "bt"), ("bf16", "plain"), ("bf16", "bt")])
+def test_tile_and_slice_edges(hb, kind, layout, m, k, n):
+    g = rng(8800 + m + k + n)
+    alpha, beta = [(1.0, 0.0), (-0.75, 0.3)][(m + k) % 2]
+    _check(hb, kind, layout, g.standard_normal((m, k)), g.standard_normal((k, n)),
+           g.standard_normal((m, n)), m, k, n, alpha, beta)
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_negative_zero_sums_survive_the_padding(hb, kind):
+    m, k, n = 40, 19, 36
+    a, b, c = -np.zeros((m, k), np.float32), np.ones((k, n), np.float32), -np.zeros((m, n), np.float32)
+    _check(hb, kind, "plain", a, b, c, m, k, n, 1.0, 1.0)
+
+
+@pytest.mark.parametrize("alpha", [1.0, 2.0 ** -10, 1.9921875, 0.3])
+@pytest.mark.parametrize("low,high", [(-126, -60), (-70, 70), (60, 127), (-56, -54), (61, 63)])
+def test_bf16_exponents_whose_products_round(hb, alpha, low, high):
+    """Products that underflow, overflow or lose bits keep their own rounding, a factor 2^(low..high)
+    on either side, in one tile of several and in a last slice that is not full."""
+    m, k, n = 70, 75, 100
+    g = rng(8900 + low + high)
+    a, b = g.standard_normal((m, k)), g.standard_normal((k, n))
+    at = (g.integers(0, m, 40), g.integers(0, k, 40))
+    a[at] = np.ldexp(a[at], g.integers(low, high + 1, 40))
+    a[5] = np.ldexp(a[5], g.integers(low, high + 1, k))
+    bt = (g.integers(0, k, 40), g.integers(0, n, 40))
+    b[bt] = np.ldexp(b[bt], g.integers(low, high + 1, 40))
+    with np.errstate(over="ignore"):
+        _check(hb, "bf16", "bt", a, b, g.standard_normal((m, n)), m, k, n, alpha, 0.5)
