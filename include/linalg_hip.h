@@ -449,9 +449,10 @@ typedef struct lg_contract_plan {
                              (2 for 128x128 tiles, 4 for 64x64); LG_KERNEL_PIPELINED on 64x64
                              tiles: 4 (each wave takes a quarter of every K chunk); else 1 */
     uint32_t reserved;
-    /* f32 plans of tiles of 128x128 and more with K chunks of at least 64 keep their tiles, grid and
+    /* f32 plans of 64x64 tiles and more with long enough K chunks keep their tiles, grid and
      * splits but multiply on the bf16 matrix cores, every element as three bf16 pieces that
-     * hold it whole (csrc/gemm_split.h); the launch log names the kernel gemm_f32_b3. */
+     * hold it whole (csrc/gemm_split.h); the launch log names the kernel gemm_f32_b3*. There a
+     * 64x64 tile has kgroups 4, and a 128x128 one one wave group whatever kgroups says. */
 } lg_contract_plan;
 
 lg_status lg_plan_contract_f32(float alpha, const lg_view* a, const char* a_labels,

@@ -12,9 +12,10 @@
 // operations in this order; the file is compiled with -ffp-contract=off, so no multiply and add
 // fuse. alpha * widen(a) does not depend on the column, so it is formed once per A element as
 // the slice is staged: the same rounding the loop performs at every use. That leaves one
-// multiply and one add per term, on the VALU (the f32 matrix cores sum in their own order).
+// multiply and one add per term: fused on the f32 matrix cores where the product needs no rounding
+// (gemm16_chain, below), else separate on the VALU (gemm16_seq).
 //
-// Tiling: 128x128 outputs per 256-thread workgroup, 8x8 per thread as two 4-row by two
+// gemm16_seq's tiling: 128x128 outputs per 256-thread workgroup, 8x8 per thread as two 4-row by two
 // 4-column blocks 64 apart, so each k costs a thread four 128-bit LDS reads (a wave's reads
 // are 4 broadcast addresses of A and 16 consecutive 16-byte words of B: no bank conflicts) for
 // 128 VALU operations; 64x64 tiles (4x4 per thread, two reads for 32 operations) where the

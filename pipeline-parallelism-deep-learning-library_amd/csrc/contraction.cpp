@@ -416,14 +416,23 @@ int load_mode_half(uintptr_t base, uint64_t off, uint64_t sb, uint64_t srow, uin
 }
 
 // Whether a tiled plan runs on the bf16 matrix cores with every element in three pieces
-// (gemm_split.h): the tiles of 128x128 and more, K chunks long enough to fill its pipeline, at least the four
-// rows and columns a thread loads at once, and operand tiles whose elements lie within 32 bits of
-// bytes of their first one, which is how the kernel addresses them.
-bool pieces_fit(const GemmArgs& t) {
-    if (t.kernel != KERN_TILE && t.kernel != KERN_DIRECT && t.kernel != KERN_PIPE) return false;
-    if (t.tile < GEMM_BM || t.tile_n < GEMM_BN || t.kgroups != 1) return false;
-    const uint32_t last = t.k - (t.splits - 1) * t.k_chunk;
+// (gemm_split.h): K chunks long enough to fill its pipeline, at least the four rows and columns a
+// thread loads at once, and operand tiles whose elements lie within 32 bits of bytes of their
+// first one, which is how the kernel addresses them. 64x64 tiles convert twice as much per product and keep
+// the f32 matrix instruction for short chunks (us, f32 against pieces): split 128 deep 13.6 against
+// 14.0 (200 x 190 x 2000), 512 deep 51 against 35 (1984 x 128 x 4928); operands with aligned unit-stride axes 336 deep 31
+// against 31 (17 x 880 x 176), 1008 deep 90 against 81 (12 x 896 x 368); and whole K over four
+// wave groups with A along K 28.8 against 29.5 (1024 x 1024 x 1000), A along M 40 against 30.
+bool pieces_fit(const GemmArgs& t, int a_mode, int b_mode) {
+    if (t.kernel != KERN_TILE && t.kernel != KERN_DIRECT && t.kernel != KERN_PIPE && t.kernel != KERN_SK) return false;
+    if (t.tile < GEMM_SMALL_TILE || (t.tile != PIPE_TALL_M && t.tile_n < t.tile)) return false;
+        const uint32_t last = t.k - (t.splits - 1) * t.k_chunk;
     if (std::min(t.k_chunk, last) < PIECES_MIN_K || t.m < 4 || t.n < 4) return false;
+    if (t.tile == GEMM_SMALL_TILE) {
+        const bool aligned = a_mode != LOAD_S && b_mode != LOAD_S;
+        if (t.k_chunk < (aligned ? 512u : 256u)) return false;
+        if (t.kernel == KERN_DIRECT && a_mode == LOAD_K) return false;
+    }
     auto near = [](uint64_t rows, int64_t srow, int64_t sk) {
         const uint64_t limit = 1ull << 29;  // elements, half of 2^32 bytes
         const uint64_t r = static_cast<uint64_t>(srow), k = static_cast<uint64_t>(sk);
@@ -796,6 +805,8 @@ Plan plan_merged(const View& a, const View& b, const View& c, const Merged& mg, 
     auto grid_of = [&](uint32_t e) {
         return static_cast<uint64_t>((mm + e - 1) / e) * ((nn + e - 1) / e) * batch;
     };
+    const int a_mode = load_mode(ra.base, ra.offset, ra.sb, ra.srow, ra.sk);
+    const int b_mode = load_mode(rb.base, rb.offset, rb.sb, rb.srow, rb.sk);
     const uint64_t useful = static_cast<uint64_t>(mm) * nn * batch;
     const uint64_t big = grid_of(GEMM_BM), mid = grid_of(GEMM_SMALL_TILE), tiny = grid_of(GEMM_TINY_TILE);
     const uint64_t k_ways = std::max<uint64_t>(1, std::min<uint64_t>(k / SPLIT_MIN_CHUNK, SPLIT_MAX));
@@ -811,7 +822,11 @@ Plan plan_merged(const View& a, const View& b, const View& c, const Merged& mg, 
         // instead. The constant is the part's; plans depend on the shape alone.
         const uint64_t rounds_big = (big + GEMM_CUS - 1) / GEMM_CUS;
         const uint64_t rounds_mid = (mid + GEMM_CUS - 1) / GEMM_CUS;
-        const bool uneven = big >= GEMM_CUS && 20 * rounds_mid < 68 * rounds_big;
+        // Operands without aligned unit-stride axes keep the large tile where the three-piece
+        // kernel takes them: it converts half as much per product (3001 x 2011 x 1537, 384 tiles:
+        // 151 us against 164 on 64x64 tiles; 459 on those with the f32 instruction).
+        const bool strided = (a_mode == LOAD_S || b_mode == LOAD_S) && k >= PIECES_MIN_K;
+        const bool uneven = big >= GEMM_CUS && 20 * rounds_mid < 68 * rounds_big && !strided;
         // A 128x128 grid that would need split-K to fill the chip takes 64x64 tiles when those
         // alone fill it in (nearly) whole rounds and K is short, so the split chunks would be
         // only a few slices deep (1024^3: 64 tiles split 8 ways, 54 TFLOP/s; 256 64x64 tiles,
@@ -829,8 +844,6 @@ Plan plan_merged(const View& a, const View& b, const View& c, const Merged& mg, 
         t.tile = GEMM_TINY_TILE;
         t.kernel = tiny >= WAVE_MIN_TILES ? KERN_WAVE : KERN_SMALL;
     }
-    const int a_mode = load_mode(ra.base, ra.offset, ra.sb, ra.srow, ra.sk);
-    const int b_mode = load_mode(rb.base, rb.offset, rb.sb, rb.srow, rb.sk);
     info.a_mode = static_cast<uint32_t>(a_mode);
     info.b_mode = static_cast<uint32_t>(b_mode);
     t.tile_n = t.tile;
@@ -1017,7 +1030,9 @@ Plan plan_merged(const View& a, const View& b, const View& c, const Merged& mg, 
     }
     t.splits = splits;
     t.k_chunk = chunk;
-    t.pieces = pieces_fit(t) ? 1 : 0;
+    t.pieces = pieces_fit(t, a_mode, b_mode) ? 1 : 0;
+    // The three-piece kernel's four waves split K on every 64x64 tile.
+    if (t.pieces != 0 && t.tile == GEMM_SMALL_TILE) t.kgroups = PIPE_KW;
     info.kgroups = t.kgroups;
     info.kernel = t.kernel == KERN_SK       ? LG_KERNEL_STREAMK
                   : t.kernel == KERN_TILE   ? LG_KERNEL_TILE

@@ -18,7 +18,7 @@
 
 #include <type_traits>
 
-#include "gemm_dlds.h"
+#include "gemm_pipe.h"
 
 namespace lg {
 namespace gemm_detail {
@@ -173,7 +173,7 @@ struct B3Loader {
             }
         }
     }
-    __device__ __forceinline__ void advance() { base += B3_BK * sk; }
+    __device__ __forceinline__ void advance(int slices = 1) { base += slices * B3_BK * sk; }
 
     // Row i of the block: its pieces into a stage.
     template <bool SCALE>
@@ -414,6 +414,30 @@ __device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const
     }
 }
 
+// A tile's sums over k [0, klen), by whichever way holds its elements.
+template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
+__device__ __forceinline__ void b3_sums(const GemmArgs& p, char* smem, const float* A, const float* B, uint32_t m0,
+                                        uint32_t n0, uint32_t klen, int wave, int lane, floatx16 (&acc)[FM][FN]) {
+    const bool bad = b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, acc);
+    // x * 0 is 0 unless x is infinite or NaN. Rows and columns past the output's edge hold
+    // whatever the stages held, and do not count.
+    const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
+    float z = 0.0f;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float t = acc[i][j][r] * 0.0f;
+                if (!EDGE || (m0 + (wm * FM + i) * 32 + (r >> 2) * 8 + h * 4 + (r & 3) < p.m &&
+                              n0 + (wn * FN + j) * 32 + lr < p.n)) {
+                    z = z + t;
+                }
+            }
+    if (__syncthreads_or(bad || z != 0.0f)) b3_redo<FM, FN, WN>(p, A, B, m0, n0, klen, wave, lane, acc);
+}
+
 // gemm_f32_b3<AM, BMD, WM, WN, FM, FN, EDGE>: C = beta * C + sum_k (alpha * a) * b, or raw split-K partials,
 // on (32 FM WM) x (32 FN WN) tiles of WM x WN waves: 256x256 and 256x128 and 128x256 tiles with eight waves
 // (the first with 4 x 2 blocks each, so that a piece read from LDS feeds twice the products), 128x128 with
@@ -443,25 +467,8 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
     const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
     floatx16 acc[FM][FN];
     b3_zero(acc);
-    bool bad = b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, acc);
-    // x * 0 is 0 unless x is infinite or NaN. Rows and columns past the output's edge hold
-    // whatever the stages held, and do not count.
+    b3_sums<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, wave, lane, acc);
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
-    float z = 0.0f;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float t = acc[i][j][r] * 0.0f;
-                if (!EDGE || (m0 + (wm * FM + i) * 32 + (r >> 2) * 8 + h * 4 + (r & 3) < p.m &&
-                              n0 + (wn * FN + j) * 32 + lr < p.n)) {
-                    z = z + t;
-                }
-            }
-    if (__syncthreads_or(bad || z != 0.0f)) b3_redo<FM, FN, WN>(p, A, B, m0, n0, klen, wave, lane, acc);
-
     float* C = p.partial != nullptr ? p.partial + static_cast<int64_t>(plane) * p.m * p.n
                                     : p.c + static_cast<int64_t>(bi) * p.c_sb;
     const int64_t c_sm = p.partial != nullptr ? static_cast<int64_t>(p.n) : p.c_sm;
@@ -482,6 +489,254 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
                 *q = v;
             }
         }
+}
+
+// gemm_f32_b3kw<AM, BMD, EDGE>: a 64x64 tile per workgroup, each of four waves summing the whole tile
+// over every fourth slice of the K chunk, for outputs of too few 128x128 tiles, or tiles that would spread
+// unevenly. A wave's 2 x 2 blocks then read 12 fragments for 24 MFMAs, as 128x128 tiles do (waves
+// of 32x32 sharing stages would read twice that, the LDS's whole rate), and nothing but its own loads
+// and LDS accesses, which complete in order, holds it: no barrier before the end, one stage a wave. The price is the
+// conversion, once per wave: 208 VALU instructions for 24 MFMAs, more than they hide, so two workgroups
+// share a compute unit. The sums meet in LDS as (s0 + s1) + (s2 + s3), each wave storing one block. Bound:
+// the VALU, at 110-115 TFLOP/s. Against the f32 instruction: 3001 x 2011 x 1537 with odd rows 459 -> 164 us
+// (32-bit loads before), 2300 x 2304 x 2304 274 -> 219, 320 x 352 x 97536 418 -> 224, 37^6 in rank 4 147 -> 56,
+// 256 x 256 x 65536 77.4 -> 75.5.
+template <int AM, int BMD, bool EDGE>
+__global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
+    constexpr int R = 64, W = 4;
+    using G = B3Geo<R>;
+    constexpr int ST = 2 * G::BYTES;
+    // The stages, then the four sums: two workgroups per compute unit.
+    constexpr int SM = W * (ST > R * R * 4 ? ST : R * R * 4);
+    static_assert(SM <= 80 * 1024, "two workgroups per compute unit");
+    __shared__ __attribute__((aligned(16))) char smem[SM];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 31, h = lane >> 5;
+    uint32_t plane, tm, tn;
+    decode_tile(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, &plane, &tm, &tn);
+    const uint32_t bi = plane / p.splits, split = plane - bi * p.splits;
+    const uint32_t m0 = tm * R, n0 = tn * R, kb = split * p.k_chunk;
+    const uint32_t klen = min(p.k - kb, p.k_chunk);
+    const float* A = p.a + static_cast<int64_t>(bi) * p.a_sb + static_cast<int64_t>(kb) * p.a_sk;
+    const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
+    char* mine = smem + wave * ST;
+    const char* fa = mine + (lane & 3) * G::CLS + (lr >> 2) * 16 + h * G::CH;
+    const char* fb = fa + G::BYTES;
+
+    // This wave's slices: wave, wave + 4, ...; the chunk's last may hold `left` < 16 k.
+    const uint32_t total = (klen + B3_BK - 1) / B3_BK, left = klen % B3_BK;
+    const uint32_t slices = (total - wave + W - 1) / W;
+    const bool tail = EDGE && left != 0 && (total - 1) % W == static_cast<uint32_t>(wave);
+    B3Loader<AM, R, EDGE> la;
+    B3Loader<BMD, R, EDGE> lb;
+    la.init(A, p.a_sm, p.a_sk, m0, p.m, lane);
+    lb.init(B, p.b_sn, p.b_sk, n0, p.n, lane);
+    la.advance(wave);
+    lb.advance(wave);
+    const float alpha_a = p.scale_b ? 1.0f : p.alpha, alpha_b = p.scale_b ? p.alpha : 1.0f;
+    floatx16 acc[2][2];
+    b3_zero(acc);
+    B3Low low;
+    auto loop = [&](auto scaled) __attribute__((always_inline)) {
+        constexpr bool SCALE = decltype(scaled)::value;
+        B3Block xa[2], xb[2];
+        auto fetch = [&](uint32_t s, int to) __attribute__((always_inline)) {
+            if (s != 0 && s < slices) {
+                la.advance(W);
+                lb.advance(W);
+            }
+            if (EDGE && tail && s + 1 >= slices) {
+                la.load_tail(xa[to], left);
+                lb.load_tail(xb[to], left);
+            } else {
+                la.load(xa[to]);
+                lb.load(xb[to]);
+            }
+        };
+        auto put = [&](int from) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                la.template store_row<SCALE>(mine, xa[from], r, alpha_a, low);
+                lb.template store_row<SCALE>(mine + G::BYTES, xb[from], r, alpha_b, low);
+            }
+        };
+        // Other lanes read what a lane wrote: the compiler keeps their order, the LDS does by itself.
+        auto in_order = [] { __asm__ volatile("" ::: "memory"); };
+        auto step = [&](auto phase, uint32_t s) __attribute__((always_inline)) {
+            constexpr int U = decltype(phase)::value;
+            bf16x8 a[2][3], b[2][3];
+            in_order();
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    a[i][q] = *reinterpret_cast<const bf16x8*>(fa + q * G::PL + i * 128);
+                    b[i][q] = *reinterpret_cast<const bf16x8*>(fb + q * G::PL + i * 128);
+                }
+            in_order();
+            put(U ^ 1);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) b3_block<2>(a[i], b, acc[i], [](int) {});
+#pragma unroll
+            for (int q = 0; q < 24; ++q) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(s + 3, U ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        fetch(0, 0);
+        fetch(1, 1);
+        put(0);
+        fetch(2, 0);
+        uint32_t s = 0;
+        for (; s + 1 < slices; s += 2) {
+            step(std::integral_constant<int, 0>{}, s);
+            step(std::integral_constant<int, 1>{}, s + 1);
+        }
+        if (s < slices) step(std::integral_constant<int, 0>{}, s);
+    };
+    if (p.alpha != 1.0f) loop(std::true_type{});
+    else loop(std::false_type{});
+
+    const bool tiny = __syncthreads_or(low.tiny());
+    {
+        float* q = reinterpret_cast<float*>(smem) + wave * (R * R) + lane;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) q[((i * 2 + j) * 16 + r) * 64] = acc[i][j][r];
+    }
+    __syncthreads();
+    const int bm = wave >> 1, bn = wave & 1;
+    const uint32_t col = n0 + bn * 32 + lr;
+    auto row_of = [&](int r) { return m0 + bm * 32 + (r >> 2) * 8 + h * 4 + (r & 3); };
+    floatx16 v[1][1];
+    float z = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float* q = reinterpret_cast<const float*>(smem) + (wave * 16 + r) * 64 + lane;
+        v[0][0][r] = (q[0] + q[R * R]) + (q[2 * R * R] + q[3 * R * R]);
+        const float t = v[0][0][r] * 0.0f;
+        if (!EDGE || (row_of(r) < p.m && col < p.n)) z = z + t;
+    }
+    // (Each wave's own block, over the whole chunk.)
+    if (__syncthreads_or(tiny || z != 0.0f)) b3_redo<1, 1, 2>(p, A, B, m0, n0, klen, wave, lane, v);
+    float* C = p.partial != nullptr ? p.partial + static_cast<int64_t>(plane) * p.m * p.n
+                                    : p.c + static_cast<int64_t>(bi) * p.c_sb;
+    const int64_t c_sm = p.partial != nullptr ? static_cast<int64_t>(p.n) : p.c_sm;
+    const int64_t c_sn = p.partial != nullptr ? 1 : p.c_sn;
+    const float beta = p.partial != nullptr ? 0.0f : p.beta;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        if (EDGE && (row_of(r) >= p.m || col >= p.n)) continue;
+        float* q = C + row_of(r) * c_sm + col * c_sn;
+        float x = v[0][0][r];
+        if (beta != 0.0f) x = beta * *q + x;
+        *q = x;
+    }
+}
+
+// gemm_f32_b3sk<AM, BMD>: gemm_f32_sk's runs, slots and tickets (gemm_pipe.h) over the three-piece
+// sums of full 128x128 tiles: each run's part of a tile is checked, and summed again where it must be, before
+// it meets the other run's. One workgroup per compute unit. 48^6 in rank 4 (2304^3): 185 -> 149 us, 164 TFLOP/s,
+// with one wave per SIMD; 2048^3, the same wave on whole tiles, 126 -> 98 us.
+template <int AM, int BMD>
+__global__ __launch_bounds__(256, 1) void gemm_f32_b3sk(GemmArgs p) {
+    constexpr int FM = 2, FN = 2, RA = 128, RB = 128, SLOT = 128 * 128, STEP = 128;
+    constexpr int ST = B3Geo<RA>::BYTES + B3Geo<RB>::BYTES;
+    __shared__ __attribute__((aligned(16))) char smem[2 * ST + 16];
+    uint32_t& ticket = *reinterpret_cast<uint32_t*>(smem + 2 * ST);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    const uint32_t G = gridDim.x, bid = blockIdx.x;
+    const uint32_t xcd = bid & 7u, slot_in = bid >> 3, q8 = G >> 3, r8 = G & 7u;
+    const uint32_t r = xcd < r8 ? xcd * (q8 + 1) + slot_in : r8 * (q8 + 1) + (xcd - r8) * q8 + slot_in;
+    const uint32_t per_plane = p.tiles_m * p.tiles_n;
+    const uint64_t T = static_cast<uint64_t>(per_plane) * p.batch;
+    const uint32_t S = p.k / STEP;
+    const uint64_t steps = T * S;
+    uint64_t x = static_cast<uint64_t>(r) * steps / G;
+    const uint64_t end = static_cast<uint64_t>(r + 1) * steps / G;
+
+    while (x < end) {
+        const uint64_t t = x / S;
+        const uint32_t s0 = static_cast<uint32_t>(x - t * S);
+        const uint32_t s1 = static_cast<uint32_t>(min(static_cast<uint64_t>(S), s0 + (end - x)));
+        const uint32_t len = s1 - s0;
+        const bool whole = len == S;
+        const bool first_part = s0 > 0;            // the run started inside this tile
+        const uint32_t b = first_part ? r : r + 1;  // the run boundary splitting the tile
+        const uint32_t k0 = whole || first_part ? 0 : S - len;
+        const uint32_t bi = static_cast<uint32_t>(t / per_plane);
+        const uint32_t tp = static_cast<uint32_t>(t - static_cast<uint64_t>(bi) * per_plane);
+        const uint32_t group = tp / (8 * p.tiles_n), first_m = group * 8;
+        const uint32_t gm = min(p.tiles_m - first_m, 8u), in_group = tp - group * 8 * p.tiles_n;
+        const uint32_t m0 = (first_m + in_group % gm) * RA, n0 = (in_group / gm) * RB;
+        const uint32_t kb = k0 * STEP;
+        const float* A = p.a + static_cast<int64_t>(bi) * p.a_sb + static_cast<int64_t>(kb) * p.a_sk;
+        const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
+        floatx16 acc[FM][FN];
+        b3_zero(acc);
+        b3_sums<AM, BMD, 2, 2, FM, FN, false>(p, smem, A, B, m0, n0, len * STEP, wave, lane, acc);
+        if (whole) {
+            pl_store_c<FN>(p, acc, bi, m0, n0);
+        } else {
+            float* mine = p.partial + static_cast<int64_t>(2 * b + (first_part ? 1 : 0)) * SLOT + tid;
+            const float* other = p.partial + static_cast<int64_t>(2 * b + (first_part ? 0 : 1)) * SLOT + tid;
+            bool done = false;
+            if (!first_part) {
+                if (tid == 0) {
+                    ticket = __hip_atomic_load(p.counters + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                __syncthreads();
+                done = ticket == 1;  // the first part's sum is complete
+                __syncthreads();     // every thread has read `ticket` before it is reused
+            }
+            if (!done) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            __hip_atomic_store(mine + ((i * FN + j) * 16 + e) * 256, acc[i][j][e],
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+                wait_vm<0>();  // every store of this thread acknowledged
+                __syncthreads();
+                if (tid == 0) {
+                    ticket = __hip_atomic_fetch_add(p.counters + b, 1u, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+                }
+                __syncthreads();
+                done = ticket == 1;
+            }
+            if (done) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            acc[i][j][e] = acc[i][j][e] + __hip_atomic_load(other + ((i * FN + j) * 16 + e) * 256,
+                                                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+                pl_store_c<FN>(p, acc, bi, m0, n0);
+                if (tid == 0) __hip_atomic_store(p.counters + b, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        x += len;
+        // Every wave is done with the stages, and with `ticket`, before the next tile's writes.
+        wait_lgkm0();
+        __syncthreads();
+    }
 }
 
 }  // namespace gemm_detail

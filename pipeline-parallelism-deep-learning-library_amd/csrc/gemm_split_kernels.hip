@@ -22,6 +22,27 @@ void launch_tiles(hipStream_t s, const GemmArgs& a, uint32_t groups) {
     hipLaunchKernelGGL((gemm_f32_b3<AM, BMD, WM, WN, FM, FN, EDGE>), dim3(groups), dim3(64 * WM * WN), 0, s, a);
 }
 
+template <int AM, int BMD, bool EDGE>
+void launch_kw(hipStream_t s, const GemmArgs& a, uint32_t groups) {
+    if (a.tile != GEMM_SMALL_TILE || a.tile_n != GEMM_SMALL_TILE ||
+        (!EDGE && (a.m % a.tile != 0 || a.n % a.tile_n != 0 || a.k % B3_BK != 0)) ||
+        (a.k_chunk % B3_BK != 0 && a.splits > 1)) {
+        fail_invalid("three-piece GEMM launch does not match its tiles");
+    }
+    hipLaunchKernelGGL((gemm_f32_b3kw<AM, BMD, EDGE>), dim3(groups), dim3(256), 0, s, a);
+}
+
+template <int AM, int BMD>
+void launch_sk(hipStream_t s, const GemmArgs& a, uint32_t groups) {
+    const uint64_t tiles = static_cast<uint64_t>(a.tiles_m) * a.tiles_n * a.batch;
+    if (a.tile != GEMM_BM || a.tile_n != GEMM_BN || a.m % GEMM_BM != 0 || a.n % GEMM_BN != 0 || a.k % 128 != 0 ||
+        a.splits != 1 || tiles < groups || groups != SK_RANGES || a.partial == nullptr || a.counters == nullptr) {
+        fail_invalid("the stream-K GEMM needs full 128x128 tiles, at least one per range, K in whole steps "
+                     "and its scratch");
+    }
+    hipLaunchKernelGGL((gemm_f32_b3sk<AM, BMD>), dim3(groups), dim3(256), 0, s, a);
+}
+
 }  // namespace
 
 const char* launch_gemm_pieces(hipStream_t s, const GemmArgs& a, uint32_t groups) {
@@ -31,6 +52,19 @@ const char* launch_gemm_pieces(hipStream_t s, const GemmArgs& a, uint32_t groups
     if (am == AMV && bm == BMV) {                               \
         launch_tiles<AMV, BMV, __VA_ARGS__>(s, a, groups);      \
     } else
+    if (a.kernel == KERN_SK) {
+#define LG_SK(AMV, BMV, NAME)                \
+    if (am == AMV && bm == BMV) {             \
+        launch_sk<AMV, BMV>(s, a, groups);    \
+        return NAME;                          \
+    }
+        LG_SK(LOAD_K, LOAD_K, "gemm_f32_b3sk<K,K>")
+        LG_SK(LOAD_K, LOAD_MN, "gemm_f32_b3sk<K,MN>")
+        LG_SK(LOAD_MN, LOAD_K, "gemm_f32_b3sk<MN,K>")
+        LG_SK(LOAD_MN, LOAD_MN, "gemm_f32_b3sk<MN,MN>")
+#undef LG_SK
+        fail_invalid("the stream-K GEMM needs a unit-stride axis in both operands");
+    }
     if (a.tile == 256 && a.tile_n == 256) {
         LG_TILES(LOAD_K, LOAD_K, 2, 4, 4, 2, false)
         LG_TILES(LOAD_K, LOAD_MN, 2, 4, 4, 2, false) { fail_invalid("256x256 tiles need A contiguous along K"); }
@@ -47,6 +81,34 @@ const char* launch_gemm_pieces(hipStream_t s, const GemmArgs& a, uint32_t groups
         {"gemm_f32_b3<S,K>", "gemm_f32_b3<S,MN>", "gemm_f32_b3<S,S>"}};
     static const char* const wide[2][2] = {{"gemm_f32_b3_128x256<K,K>", "gemm_f32_b3_128x256<K,MN>"},
                                            {"gemm_f32_b3_128x256<MN,K>", "gemm_f32_b3_128x256<MN,MN>"}};
+    static const char* const kw[3][3] = {
+        {"gemm_f32_b3kw<K,K>", "gemm_f32_b3kw<K,MN>", "gemm_f32_b3kw<K,S>"},
+        {"gemm_f32_b3kw<MN,K>", "gemm_f32_b3kw<MN,MN>", "gemm_f32_b3kw<MN,S>"},
+        {"gemm_f32_b3kw<S,K>", "gemm_f32_b3kw<S,MN>", "gemm_f32_b3kw<S,S>"}};
+#define LG_KW(AMV, BMV, EDGEV)                      \
+    if (am == AMV && bm == BMV) {                    \
+        launch_kw<AMV, BMV, EDGEV>(s, a, groups);    \
+    } else
+    if (a.tile == GEMM_SMALL_TILE) {
+        if (full && am != LOAD_S && bm != LOAD_S) {
+            LG_KW(LOAD_K, LOAD_K, false)
+            LG_KW(LOAD_K, LOAD_MN, false)
+            LG_KW(LOAD_MN, LOAD_K, false)
+            LG_KW(LOAD_MN, LOAD_MN, false) { fail_invalid("unknown operand load mode"); }
+        } else {
+            LG_KW(LOAD_K, LOAD_K, true)
+            LG_KW(LOAD_K, LOAD_MN, true)
+            LG_KW(LOAD_MN, LOAD_K, true)
+            LG_KW(LOAD_MN, LOAD_MN, true)
+            LG_KW(LOAD_K, LOAD_S, true)
+            LG_KW(LOAD_MN, LOAD_S, true)
+            LG_KW(LOAD_S, LOAD_K, true)
+            LG_KW(LOAD_S, LOAD_MN, true)
+            LG_KW(LOAD_S, LOAD_S, true) { fail_invalid("unknown operand load mode"); }
+        }
+        return kw[am][bm];
+    }
+#undef LG_KW
     if (a.tile_n == GEMM_WIDE_N) {
         LG_TILES(LOAD_K, LOAD_K, 2, 4, 2, 2, true)
         LG_TILES(LOAD_K, LOAD_MN, 2, 4, 2, 2, true)

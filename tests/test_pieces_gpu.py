@@ -54,16 +54,24 @@ def _check(got, a, b, alpha, beta, c0):
     (2048, 2048, 80, False, False, 1),    # full tiles, five slices
     (2048, 2048, 90, True, True, 2),      # no unit stride in A
     (1921, 1925, 67, False, False, 2),
+    (3001, 2011, 77, False, True, 1),     # 384 tiles, odd rows: 128x128 all the same
+    (130, 190, 20001, False, True, 1),     # 64x64 tiles split along K, the last chunk ragged
+    (190, 130, 20011, True, False, 2),     # the same, strided, a wave with the chunk's short slice
+    (1000, 1020, 1537, True, True, 1),    # 64x64 tiles, whole K, A along M
+    (2300, 2304, 520, False, False, 1),   # 64x64 tiles of an uneven grid
+    (2304, 2304, 256, True, True, 1),     # stream-K
 ])
 @pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (-0.3, 0.75)])
 def test_tile_edges(ctx, pool, m, n, k, ta, tb, stride, alpha, beta):
     g = rng(9100 + m + n + k)
+    kernel = {130: "gemm_f32_b3kw", 190: "gemm_f32_b3kw", 1000: "gemm_f32_b3kw", 2300: "gemm_f32_b3kw",
+              2304: "gemm_f32_b3sk"}.get(m, "gemm_f32_b3<")
     a = g.standard_normal((m, k)).astype(np.float32)
     b = g.standard_normal((k, n)).astype(np.float32)
     c0 = g.standard_normal((m, n)).astype(np.float32) if beta else None
     alpha = float(np.float32(alpha))
     got, name = _product(ctx, pool, a, b, ta, tb, alpha, beta, c0, stride)
-    assert name.startswith("gemm_f32_b3"), name
+    assert name.startswith(kernel), name
     _check(got, a, b, alpha, beta, c0)
 
 
@@ -81,19 +89,20 @@ def test_pieces_hold_the_element_whole(ctx, pool):
     assert np.array_equal(got, a[:, perm])
 
 
+@pytest.mark.parametrize("shape", [(2045, 1930, 77), (1000, 1020, 1537), (2304, 2304, 256)])
 @pytest.mark.parametrize("what", ["inf", "nan", "huge", "tiny", "subnormal", "zero"])
-def test_elements_outside_the_pieces(ctx, pool, what):
+def test_elements_outside_the_pieces(ctx, pool, what, shape):
     """Infinities, NaNs, elements past bf16's largest and below what three pieces hold: the
     products of f32 arithmetic, wherever in K and in the tile they stand."""
-    m, n, k = 2045, 1930, 77
+    m, n, k = shape
     g = rng(9300)
     a = g.standard_normal((m, k)).astype(np.float32)
     b = g.standard_normal((k, n)).astype(np.float32)
     if what in ("inf", "nan"):
         v = np.float32(np.inf if what == "inf" else np.nan)
-        a[5, 76], a[700, 0], a[2044, 30], b[40, 1929] = v, -v, v, v
+        a[5, k - 1], a[700, 0], a[m - 1, 30], b[40, n - 1] = v, -v, v, v
     elif what == "huge":
-        a[5, 76] = a[2044, 3] = np.finfo(np.float32).max
+        a[5, k - 1] = a[m - 1, 3] = np.finfo(np.float32).max
         b *= np.float32(2.0 ** -10)
     elif what == "tiny":
         a *= np.float32(2.0 ** -115)
@@ -105,7 +114,7 @@ def test_elements_outside_the_pieces(ctx, pool, what):
         a[701:] = 0
     else:
         a[:] = 0
-    got, name = _product(ctx, pool, a, b, False, False)
+    got, name = _product(ctx, pool, a, b, m == 1000, False)
     assert name.startswith("gemm_f32_b3"), name
     with np.errstate(invalid="ignore", over="ignore"):
         want = a.astype(np.float64) @ b.astype(np.float64)
