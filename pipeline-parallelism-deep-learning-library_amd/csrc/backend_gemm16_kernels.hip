@@ -229,10 +229,13 @@ __global__ __launch_bounds__(QT) void gemm16_seq(Gemm16SeqArgs p) {
 // threads load: each 16 k of one row, so a slice is 2048 / (32 NB) deep. Stages hold f32,
 // [16 k][k % 4][row][k / 4], so a lane's four steps are one 128-bit read, lanes on distinct banks. Two stages, the
 // loads of a slice one slice ahead of its conversion, in registers. Bound: the f32 matrix rate, 157 TFLOP/s. 2048 x 4096 x
-// 1024 against the VALU kernel gemm16_seq: bf16 411 -> 164 us, f16 411 -> 159 us; 128 x 1408 x 1024, a few
-// workgroups whose chains alone set the time, 146 -> 15 us on 32x32 tiles.
+// 1024 against the VALU kernel gemm16_seq: bf16 411 -> 156 us, f16 411 -> 159 us; 128 x 1408 x 1024, a few
+// workgroups whose chains alone set the time, 146 -> 15 us on 32x32 tiles; 1501 x 1477 x 1023 with odd rows
+// 187 -> 127 us with 16-bit loads, 66 with 128-bit ones of any alignment.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// 128 bits that are only known to be 2-byte aligned (a global load needs no more).
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2)));
 template <bool VEC>
 struct Raw16 {
     u32x4 v[2];
@@ -290,8 +293,8 @@ __global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
             const char* base = reinterpret_cast<const char*>(src + static_cast<int64_t>(s) * BK * s_k);
             if ((s + 1) * BK <= p.k) {
                 if constexpr (VEC) {
-                    x.v[0] = *reinterpret_cast<const u32x4*>(base + off);
-                    x.v[1] = *reinterpret_cast<const u32x4*>(base + 16 + off);
+                    x.v[0] = *reinterpret_cast<const u32x4u*>(base + off);
+                    x.v[1] = *reinterpret_cast<const u32x4u*>(base + 16 + off);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 16; ++j) x.v[j] = *reinterpret_cast<const uint16_t*>(base + j * s_k * 2 + off);
@@ -299,10 +302,13 @@ __global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
             } else {
                 const uint32_t k = s * BK + kg * 16;
                 if constexpr (VEC) {
-                    // Whole runs of eight: K is a multiple of eight here.
-                    x.v[0] = x.v[1] = u32x4{0, 0, 0, 0};
-                    if (k < p.k) x.v[0] = *reinterpret_cast<const u32x4*>(base + off);
-                    if (k + 8 < p.k) x.v[1] = *reinterpret_cast<const u32x4*>(base + 16 + off);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        uint32_t lo = 0, hi = 0;
+                        if (k + 2 * j < p.k) lo = *reinterpret_cast<const uint16_t*>(base + 4 * j + off);
+                        if (k + 2 * j + 1 < p.k) hi = *reinterpret_cast<const uint16_t*>(base + 4 * j + 2 + off);
+                        x.v[j >> 2][j & 3] = lo | hi << 16;
+                    }
                 } else {
 #pragma unroll
                     for (int j = 0; j < 16; ++j) {
@@ -425,11 +431,7 @@ bool chain_fuses(uint32_t kind, float alpha) {
 
 template <int HK, int NB>
 void launch_chain_nb(hipStream_t s, const Gemm16SeqArgs& a, uint32_t groups) {
-    // 128-bit loads: rows contiguous along K, 16-byte aligned, K in whole runs of eight.
-    auto vec = [&](const uint16_t* q, int64_t s_row, int64_t s_k) {
-        return s_k == 1 && s_row % 8 == 0 && a.k % 8 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0;
-    };
-    const bool av = vec(a.a, a.a_sm, a.a_sk), bv = vec(a.b, a.b_sn, a.b_sk);
+    const bool av = a.a_sk == 1, bv = a.b_sk == 1;
     const dim3 grid(groups);
     if (av && bv) hipLaunchKernelGGL((gemm16_chain<HK, NB, true, true>), grid, dim3(256), 0, s, a);
     else if (av) hipLaunchKernelGGL((gemm16_chain<HK, NB, true, false>), grid, dim3(256), 0, s, a);

@@ -23,7 +23,7 @@ def _check(hb, kind, layout, a, b, c, m, k, n, alpha, beta):
 
 
 # 128x128 tiles (529 of them, ragged), 64x64 (552) and 32x32, with K around their slices of 16, 32
-# and 64; K in whole runs of eight takes 128-bit loads.
+# and 64; rows along K are read 128 bits at a time whatever their alignment.
 @pytest.mark.parametrize("m,k,n", [(2900, 16, 2820), (2817, 17, 2944), (2823, 40, 2900), (1500, 32, 1450),
                                    (1409, 33, 1473), (1481, 104, 1472), (70, 64, 45), (33, 65, 97),
                                    (31, 1, 32), (64, 136, 64), (1, 191, 700)])
