@@ -441,7 +441,8 @@ typedef struct lg_contract_plan {
                              mostly padding;
                              32x32 for small outputs (sixteen waves per tile splitting K) and
                              batches of small products (one tile per wave); 1x1 for dot
-                             products, 1x4 for K <= 8; f16: 64x64 */
+                             products, 1x4 for K <= 8; f16: 64x64, or
+                             32x32 for grids of few of those */
     uint32_t kernel;      /* lg_plan_kernel */
     uint32_t swapped;     /* 1 when C is contiguous along M and is computed as C^T = B^T.A^T */
     uint32_t kgroups;     /* LG_KERNEL_DIRECT: wave groups per workgroup splitting the tile's K

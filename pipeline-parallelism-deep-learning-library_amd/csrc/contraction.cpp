@@ -392,6 +392,9 @@ Axes4 pack(const std::vector<Axis>& axes, char which) {
     return out;
 }
 
+// Compute units of one MI355X, for the tile-size choice only.
+constexpr uint64_t GEMM_CUS = 256;
+
 struct Plan {
     lg_contract_plan info{};
     bool half = false;  // f16 operands: the h* argument blocks below are the live ones
@@ -512,15 +515,24 @@ void plan_half(const View& a, const View& b, const View& c, const Merged& mg, fl
     t.n = n;
     t.k = k;
     t.batch = batch;
-    t.tiles_m = (m + HGEMM_BM - 1) / HGEMM_BM;
-    t.tiles_n = (n + HGEMM_BN - 1) / HGEMM_BN;
-    info.tile_m = HGEMM_BM;
-    info.tile_n = HGEMM_BN;
     info.a_mode = static_cast<uint32_t>(load_mode_half(a.base, a.offset, ab.a, am.a, ak.a));
     info.b_mode = static_cast<uint32_t>(load_mode_half(b.base, b.offset, ab.b, an.b, ak.b));
     t.alpha = alpha;
     t.beta = beta;
-    const uint64_t wg = gemm_half_workgroups(m, n, batch);
+    // The tile kernel wants whole tiles and slices of aligned operands, two workgroups of them per compute unit;
+    // everything else whose rows lie within 32 bits of bytes goes to gemm_f16_edge, on 32x32 tiles
+    // where 64x64 ones would be fewer than that and K is at least one slice.
+    auto near = [](uint64_t s_row, uint64_t s_k) { return s_row < (1u << 22) && s_k < (1u << 22); };
+    const uint64_t big = gemm_half_workgroups(m, n, batch, HGEMM_BM);
+    const bool whole = m % HGEMM_BM == 0 && n % HGEMM_BN == 0 && k % HGEMM_BK == 0 &&
+                       info.a_mode != LG_LOAD_STRIDED && info.b_mode != LG_LOAD_STRIDED;
+    const bool few = big < 2 * GEMM_CUS && k >= HGEMM_BK;
+    t.edge = (!whole || few) && near(am.a, ak.a) && near(an.b, ak.b) ? 1 : 0;
+    t.tile = t.edge != 0 && few ? 32 : HGEMM_BM;
+    t.tiles_m = (m + t.tile - 1) / t.tile;
+    t.tiles_n = (n + t.tile - 1) / t.tile;
+    info.tile_m = info.tile_n = t.tile;
+    const uint64_t wg = gemm_half_workgroups(m, n, batch, t.tile);
     if (wg > 0x7fffffffull) fail_invalid("problem exceeds one launch's workgroup count");
     info.kind = LG_PLAN_TILED;
     info.workgroups = wg;
@@ -603,8 +615,6 @@ void dot_split_shape(uint32_t batch, uint32_t k, uint32_t* splits, uint32_t* chu
     *splits = static_cast<uint32_t>((k + c - 1) / c);
 }
 
-// Compute units of one MI355X, for the tile-size choice only.
-constexpr uint64_t GEMM_CUS = 256;
 // K elements per chunk below which two wave groups would each get too few slices to pipeline.
 constexpr uint32_t KG_MIN_CHUNK = 256;
 // Longest K for which 64x64 tiles replace a split 128x128 grid.

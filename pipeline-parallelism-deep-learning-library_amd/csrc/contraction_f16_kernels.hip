@@ -9,6 +9,8 @@
 // the exact value, which is also what the reference's double-float path returns.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gemm_kernel.h"
 #include "lg_internal.h"
 
@@ -228,6 +230,206 @@ __global__ __launch_bounds__(HT, 4) void gemm_f16_f64mfma(GemmHalfArgs p) {
             }
 }
 
+// gemm_f16_edge<TILE, AV, BV>: the same product for what the kernel above serves badly: grids of
+// few 64x64 tiles, and operands or tiles whose runs of eight halves are not all inside and aligned (its
+// loads are then 16 bits each, behind predicates that keep one in flight). Loads go by rows: a thread
+// takes 16 k of one row, as two 128-bit loads (AV, BV: rows along K, of any alignment) or 16 16-bit ones,
+// consecutive lanes on consecutive rows; rows past the edge repeat the last one, so nothing is predicated
+// but a last slice. Stages are always [row][k], so a fragment is one 64-bit read whatever the operand's order.
+// TILE 64: four waves of 2 x 2 blocks in 2 x 2. TILE 32: each wave sums the whole 32x32 tile over its
+// 16 of a slice's 64 k, and the four sums are added in wave order through LDS: four times the
+// workgroups, for chains a quarter as long. Bound: the f64 matrix rate, 78.6 TFLOP/s, and for few tiles the chains.
+// us, before -> after: 247 x 527 x 1168 86 -> 18, 526 x 444 x 647 54 -> 18, 622 x 1663 x 2279 (both operands along
+// M/N) 229 -> 192 on 32x32 tiles; 1688 x 1400 x 1394 213 -> 159, 2501 x 2499 x 2001 592 -> 529 on 64x64.
+// Eight halves that are only known to be 2-byte aligned (a global load needs no more).
+typedef uint16_t h8u __attribute__((ext_vector_type(8), aligned(2)));
+template <bool VEC>
+struct HRun {
+    h8 v[2];
+};
+template <>
+struct HRun<false> {
+    uint16_t v[16];
+};
+
+template <int TILE, bool AV, bool BV>
+__global__ __launch_bounds__(HT, 4) void gemm_f16_edge(GemmHalfArgs p) {
+    constexpr int BK = 64, ST = TILE * HP;        // halves per operand stage
+    constexpr int UNITS = TILE * BK / 16;          // (row, 16 k) units of one operand's slice
+    constexpr bool BOTH = UNITS == HT;             // every thread loads a unit of each operand
+    static_assert(BOTH || 2 * UNITS == HT, "units divide over the threads");
+    constexpr int SUMS = TILE == 32 ? 4 * 32 * 32 * 8 : 0;
+    constexpr int BYTES = 4 * ST * 2 > SUMS ? 4 * ST * 2 : SUMS;
+    __shared__ __attribute__((aligned(16))) char smem[BYTES];
+    uint16_t* const stages = reinterpret_cast<uint16_t*>(smem);  // [2][A, B][TILE][HP]
+    uint32_t plane, tm, tn;
+    gemm_detail::decode_tile(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, &plane, &tm, &tn);
+    const uint32_t m0 = tm * TILE, n0 = tn * TILE;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const uint16_t* A = p.a + static_cast<int64_t>(plane) * p.a_sb + static_cast<int64_t>(m0) * p.a_sm;
+    const uint16_t* B = p.b + static_cast<int64_t>(plane) * p.b_sb + static_cast<int64_t>(n0) * p.b_sn;
+    uint16_t* C = p.c + static_cast<int64_t>(plane) * p.c_sb;
+
+    f64x4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+
+    // One operand's unit of this thread.
+    struct Unit {
+        const uint16_t* src;
+        int64_t s_k;
+        uint32_t off, at, kg;  // byte offset of the unit's first element, its place in a stage, its 16-k group
+    };
+    auto unit = [&](const uint16_t* src, int64_t s_row, int64_t s_k, uint32_t rows, uint32_t t) {
+        Unit u;
+        const bool along_k = s_k == 1;
+        const uint32_t row = along_k ? t / 4 : t % TILE;
+        u.kg = along_k ? t % 4 : t / TILE;
+        u.src = src;
+        u.s_k = s_k;
+        u.off = static_cast<uint32_t>(min(row, rows - 1) * s_row + u.kg * 16 * s_k) * 2u;
+        u.at = row * HP + u.kg * 16;
+        return u;
+    };
+    auto load = [&](auto& x, const Unit& u, uint32_t s) __attribute__((always_inline)) {
+        constexpr bool VEC = std::is_same_v<std::remove_reference_t<decltype(x)>, HRun<true>>;
+        const char* base = reinterpret_cast<const char*>(u.src + static_cast<int64_t>(s) * BK * u.s_k);
+        const uint32_t k = s * BK + u.kg * 16;
+        const bool full = (s + 1) * BK <= p.k;
+        if constexpr (VEC) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (full || k + 8 * q + 8 <= p.k) {
+                    x.v[q] = *reinterpret_cast<const h8u*>(base + 16 * q + u.off);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        x.v[q][e] = 0;
+                        if (k + 8 * q + e < p.k) x.v[q][e] = *reinterpret_cast<const uint16_t*>(base + 16 * q + 2 * e + u.off);
+                    }
+                }
+            }
+        } else if (full) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) x.v[j] = *reinterpret_cast<const uint16_t*>(base + j * u.s_k * 2 + u.off);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                x.v[j] = 0;
+                if (k + j < p.k) x.v[j] = *reinterpret_cast<const uint16_t*>(base + j * u.s_k * 2 + u.off);
+            }
+        }
+    };
+    auto put = [&](const auto& x, const Unit& u, uint16_t* st) __attribute__((always_inline)) {
+        constexpr bool VEC = std::is_same_v<std::remove_cv_t<std::remove_reference_t<decltype(x)>>, HRun<true>>;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            h8 v;
+            if constexpr (VEC) {
+                v = x.v[q];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = x.v[8 * q + e];
+            }
+            *reinterpret_cast<h8*>(st + u.at + 8 * q) = v;
+        }
+    };
+    const uint32_t slices = (p.k + BK - 1) / BK;
+    auto multiply = [&](uint32_t s) __attribute__((always_inline)) {
+        const uint16_t* as = stages + (s & 1) * 2 * ST;
+        const uint16_t* bs = as + ST;
+        const int wr = TILE == 64 ? (wave >> 1) * 32 : 0, wc = TILE == 64 ? (wave & 1) * 32 : 0;
+        auto group = [&](int q) __attribute__((always_inline)) {
+            double av[2][4], bv[2][4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) hval4<LOAD_K>(av[i], as, wr + i * 16 + li, q * 16 + lk * 4);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) hval4<LOAD_K>(bv[j], bs, wc + j * 16 + li, q * 16 + lk * 4);
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i][st], bv[j][st], acc[i][j], 0, 0, 0);
+        };
+        if constexpr (TILE == 64) {
+#pragma unroll 1
+            for (int q = 0; q < 4; ++q) group(q);
+        } else {
+            group(wave);
+        }
+    };
+    // A slice's loads go out one slice ahead of its conversion, two of its products.
+    auto run = [&](auto& x, auto& y, const Unit& u, const Unit& v, bool first, bool second) __attribute__((always_inline)) {
+        auto load_all = [&](uint32_t s) __attribute__((always_inline)) {
+            if (first) load(x, u, s);
+            if (second) load(y, v, s);
+        };
+        auto put_all = [&](uint32_t s) __attribute__((always_inline)) {
+            if (first) put(x, u, stages + (s & 1) * 2 * ST);
+            if (second) put(y, v, stages + (s & 1) * 2 * ST + ST);
+        };
+        load_all(0);
+        put_all(0);
+        if (slices > 1) load_all(1);
+        __syncthreads();
+        for (uint32_t s = 0; s < slices; ++s) {
+            if (s + 1 < slices) put_all(s + 1);
+            if (s + 2 < slices) load_all(s + 2);
+            multiply(s);
+            __syncthreads();
+        }
+    };
+    HRun<AV> xa;
+    HRun<BV> xb;
+    const uint32_t t = BOTH ? tid : tid % UNITS;
+    const Unit ua = unit(A, p.a_sm, p.a_sk, p.m - m0, t), ub = unit(B, p.b_sn, p.b_sk, p.n - n0, t);
+    if constexpr (BOTH) run(xa, xb, ua, ub, true, true);
+    else if (wave < 2) run(xa, xb, ua, ub, true, false);
+    else run(xa, xb, ua, ub, false, true);
+
+    if constexpr (TILE == 32) {
+        // Wave w keeps block (w / 2, w % 2) of the four sums.
+        double* sums = reinterpret_cast<double*>(smem);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) sums[((wave * 4 + i * 2 + j) * 4 + v) * 64 + lane] = acc[i][j][v];
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            double r = sums[(wave * 4 + v) * 64 + lane];
+#pragma unroll
+            for (int w = 1; w < 4; ++w) r = r + sums[((w * 4 + wave) * 4 + v) * 64 + lane];
+            const uint32_t row = m0 + (wave >> 1) * 16 + v * 4 + lk, col = n0 + (wave & 1) * 16 + li;
+            if (row < p.m && col < p.n) {
+                uint16_t* q = C + static_cast<int64_t>(row) * p.c_sm + static_cast<int64_t>(col) * p.c_sn;
+                *q = finish(r, p.alpha, p.beta, q);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const uint32_t row = m0 + (wave >> 1) * 32 + i * 16 + v * 4 + lk;
+                    const uint32_t col = n0 + (wave & 1) * 32 + j * 16 + li;
+                    if (row < p.m && col < p.n) {
+                        uint16_t* q = C + static_cast<int64_t>(row) * p.c_sm + static_cast<int64_t>(col) * p.c_sn;
+                        *q = finish(acc[i][j][v], p.alpha, p.beta, q);
+                    }
+                }
+    }
+}
+
 __device__ inline int64_t decode4(const Axes4& ax, uint64_t idx) {
     int64_t off = 0;
 #pragma unroll
@@ -289,13 +491,32 @@ uint32_t grid_for(uint64_t items) {
 
 }  // namespace
 
-uint64_t gemm_half_workgroups(uint32_t m, uint32_t n, uint32_t batch) {
-    return static_cast<uint64_t>((m + HGEMM_BM - 1) / HGEMM_BM) * ((n + HGEMM_BN - 1) / HGEMM_BN) * batch;
+uint64_t gemm_half_workgroups(uint32_t m, uint32_t n, uint32_t batch, uint32_t tile) {
+    return static_cast<uint64_t>((m + tile - 1) / tile) * ((n + tile - 1) / tile) * batch;
 }
+
+namespace {
+template <int TILE>
+void launch_half_edge(hipStream_t s, const GemmHalfArgs& a, dim3 grid) {
+    const bool av = a.a_sk == 1, bv = a.b_sk == 1;
+    if (av && bv) hipLaunchKernelGGL((gemm_f16_edge<TILE, true, true>), grid, dim3(HT), 0, s, a);
+    else if (av) hipLaunchKernelGGL((gemm_f16_edge<TILE, true, false>), grid, dim3(HT), 0, s, a);
+    else if (bv) hipLaunchKernelGGL((gemm_f16_edge<TILE, false, true>), grid, dim3(HT), 0, s, a);
+    else hipLaunchKernelGGL((gemm_f16_edge<TILE, false, false>), grid, dim3(HT), 0, s, a);
+}
+}  // namespace
 
 void launch_gemm_half(Context* ctx, hipStream_t s, const GemmHalfArgs& args, int a_mode,
                       int b_mode) {
-    const dim3 grid(static_cast<uint32_t>(gemm_half_workgroups(args.m, args.n, args.batch)));
+    const dim3 grid(static_cast<uint32_t>(gemm_half_workgroups(args.m, args.n, args.batch, args.tile)));
+    if (args.edge != 0) {
+        if (args.tile == 32) launch_half_edge<32>(s, args, grid);
+        else launch_half_edge<64>(s, args, grid);
+        check_hip(hipGetLastError(), "gemm_f16_edge");
+        note_launch(ctx, args.tile == 32 ? "gemm_f16_edge32" : "gemm_f16_edge");
+        return;
+    }
+    if (args.tile != HGEMM_BM) fail_invalid("the f16 tile kernel has 64x64 tiles");
 #define LG_HGEMM_CASE(AMV, BMV)                                                       \
     if (a_mode == AMV && b_mode == BMV) {                                             \
         hipLaunchKernelGGL((gemm_f16_f64mfma<AMV, BMV>), grid, dim3(HT), 0, s, args); \

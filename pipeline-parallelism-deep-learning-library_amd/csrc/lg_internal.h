@@ -272,6 +272,8 @@ struct GemmHalfArgs {
     int64_t a_sb, a_sm, a_sk, b_sb, b_sn, b_sk, c_sb, c_sm, c_sn;
     uint32_t m, n, k, batch, tiles_m, tiles_n;
     float alpha, beta;
+    uint32_t tile;  // square output tile: 64, or 32 (edge only)
+    uint32_t edge;  // 1: gemm_f16_edge
 };
 struct GeneralHalfArgs {
     const uint16_t* a;
@@ -312,7 +314,7 @@ void launch_gemm_half(Context* ctx, hipStream_t s, const GemmHalfArgs& args, int
                       int b_mode);
 void launch_general_half(Context* ctx, hipStream_t s, const GeneralHalfArgs& args);
 void launch_fill_half(Context* ctx, hipStream_t s, const FillHalfArgs& args);
-uint64_t gemm_half_workgroups(uint32_t m, uint32_t n, uint32_t batch);
+uint64_t gemm_half_workgroups(uint32_t m, uint32_t n, uint32_t batch, uint32_t tile);
 
 void launch_gemm(Context* ctx, hipStream_t s, const GemmArgs& args, int a_mode, int b_mode);
 void launch_reduce(Context* ctx, hipStream_t s, const ReduceArgs& args);

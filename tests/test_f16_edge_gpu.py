@@ -1,0 +1,36 @@
+"""The f16 contraction's edge kernel (gemm_f16_edge) around its tiles, slices and alignments.
+
+On halves of a 2^-10 grid every sum is exact in f64, so each output is the exact value rounded
+once, which numpy's float64 -> float16 conversion gives."""
+import numpy as np
+import pytest
+
+from helpers import Layout, rng
+from linalg_hip import contraction as C
+from test_contraction_f16_gpu import Half, f16_bits_equal, grid_halves
+
+pytestmark = pytest.mark.gpu
+
+
+# 32x32 tiles: one short of, at and past a tile and a slice; 64x64: K under one slice, or 552
+# ragged tiles; stride 2 leaves no unit stride, offset 1 no alignment.
+@pytest.mark.parametrize("m,n,k", [(32, 32, 64), (31, 33, 65), (65, 97, 127), (1, 700, 191), (247, 130, 128),
+                                   (70, 66, 63), (33, 40, 17), (1450, 1473, 64), (1409, 1475, 71)])
+@pytest.mark.parametrize("at,bt,stride,offset", [(False, False, 1, 0), (True, True, 1, 1), (False, True, 1, 1),
+                                                 (True, False, 2, 0)])
+def test_edges_round_once(ctx, pool, m, n, k, at, bt, stride, offset):
+    if stride == 2 and m > 1000:
+        pytest.skip("covered by the smaller shapes")
+    g = rng(8700 + m + n + k)
+    alpha, beta = [(1.0, 0.0), (0.5, -0.25)][(m + k) % 2]
+    pick = lambda t, r, c, s, o: Layout(o, [r, c], [s, r * s] if t else [c * s, s])
+    la, lb = pick(at, m, k, stride, offset), pick(bt, k, n, 1, offset)
+    a, b = Half(pool, la, grid_halves(g, la.span())), Half(pool, lb, grid_halves(g, lb.span()))
+    c0 = grid_halves(g, m * n) if beta else np.full(m * n, np.nan, np.float16)
+    c = Half(pool, Layout.dense([m, n]), c0)
+    C.gemm(ctx, alpha, a.view(), b.view(), beta, c.view())
+    assert ctx.launches()[-1].startswith("gemm_f16_edge") or m % 64 == n % 64 == k % 64 == 0
+    want = alpha * (a.logical().astype(np.float64) @ b.logical().astype(np.float64))
+    if beta:
+        want = want + beta * c0.reshape(m, n).astype(np.float64)
+    assert f16_bits_equal(c.read()[: m * n].reshape(m, n), want.astype(np.float16).view(np.uint16))
