@@ -7,7 +7,8 @@
 // b (destination unit stride). A TA x TB element tile is read with 128-bit loads running along
 // a, staged in LDS with an odd word pitch (TA*W + 1) so both the row-wise fill and the
 // column-wise drain spread over the banks, and written with 128-bit stores running along b.
-// Tiles are walked with a grid stride in the order (outer, ta, tb), tb fastest: concurrently
+// Tiles are walked with a grid stride in the order (outer, ta, tb), tb fastest (cached tiles: each
+// XCD in a run of its own): concurrently
 // running workgroups write consecutive TB-element segments of the same TA destination rows, so
 // every destination row is written front to back, and read consecutive bands of source rows.
 // (On a 1 GiB transpose this order measured 2-3% faster than ta fastest on MI355X.)
@@ -57,7 +58,18 @@ __global__ __launch_bounds__(NTH) void perm_tile(PermTileArgs p) {
     const int tid = threadIdx.x;
     const uint64_t per_outer = static_cast<uint64_t>(p.tiles_a) * p.tiles_b;
 
-    for (uint64_t t = blockIdx.x; t < p.total_tiles; t += gridDim.x) {
+    for (uint64_t lin = blockIdx.x; lin < p.total_tiles; lin += gridDim.x) {
+        // Cached tiles: workgroups are dealt to the eight XCDs in turn, and each XCD takes one
+        // contiguous run of tiles, so that the tiles on either side of a line that no tile boundary falls on
+        // (rows off the 128-byte grid) meet in one L2 instead of each moving a part of it.
+        // Measured, us: 8191 x 4099 85 -> 65, 8188 x 4100 86 -> 60, 2476 x 3864 16.8 -> 13.2, rows on the grid 4096^2
+        // 30.5 -> 29.3. Streaming tiles write whole lines past the L2 and keep the plain order (8192 x 4096
+        // 48.6 against 49.5).
+        uint64_t t = lin;
+        if constexpr (NTM == 0) {
+            const uint64_t q8 = p.total_tiles >> 3, r8 = p.total_tiles & 7u, xcd = lin & 7u;
+            t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (lin >> 3);
+        }
         uint64_t outer = t / per_outer;
         const uint64_t rem = t - outer * per_outer;
         const uint32_t ta = static_cast<uint32_t>(rem / p.tiles_b);
