@@ -1,9 +1,9 @@
 // gfx950 permutation kernels: the tiled transpose (permutation_tile.h) instantiated at the
 // library's tile geometry, and the gather copy.
 //
-// perm_copy: the destination is contiguous, so each thread produces 128 bits of it from a
-// strided gather (odometer over the source strides); a fully contiguous source is a straight
-// 128-bit copy.
+// perm_copy: the destination is contiguous, so each thread produces 128 bits of it: a straight
+// 128-bit copy of a fully contiguous source, else a strided gather (odometer over the source strides;
+// perm_rows for the ranks and sizes that occur, perm_copy for the rest).
 #include <hip/hip_runtime.h>
 
 #include "lg_internal.h"
@@ -72,6 +72,76 @@ __global__ __launch_bounds__(PERM_THREADS) void perm_copy(PermCopyArgs p) {
     }
 }
 
+// perm_copy of a gather whose rank after merging is 2 to 4 and whose elements number less than 2^32: the
+// index is decoded with 32-bit divisions into registers (perm_copy's 64-bit ones, over a rank it learns at run time,
+// bound it: 3.3 TB/s), and four neighbours of the source row, at any alignment, are one 128-bit load
+// where they lie in one row. Bound: HBM where rows are long. us, before -> after: [116,108,60,136] by 0,2,1,3
+// 249 -> 139 (5.9 TB/s), [64,128,2048] by 1,0,2 34 -> 21, [301,501,67] by 1,0,2 29 -> 19, [1000,1000,5] 42 -> 26.
+template <int W, bool CONJ, int RANK>
+__global__ __launch_bounds__(PERM_THREADS) void perm_rows(PermCopyArgs p) {
+    constexpr uint32_t VE = 4 / W;
+    const uint32_t* src = static_cast<const uint32_t*>(p.src);
+    uint32_t* dst = static_cast<uint32_t*>(p.dst) + p.dst_offset * W;
+    const uint32_t count = static_cast<uint32_t>(p.count);
+    uint32_t shape[RANK];
+#pragma unroll
+    for (int d = 0; d < RANK; ++d) shape[d] = static_cast<uint32_t>(p.shape[d]);
+    for (uint64_t at = (static_cast<uint64_t>(blockIdx.x) * PERM_THREADS + threadIdx.x) * VE; at < count;
+         at += static_cast<uint64_t>(gridDim.x) * PERM_THREADS * VE) {
+        const uint32_t i0 = static_cast<uint32_t>(at);
+        uint32_t idx[RANK], r = i0;
+        int64_t soff = static_cast<int64_t>(p.src_offset);
+#pragma unroll
+        for (int d = RANK - 1; d > 0; --d) {
+            const uint32_t q = r / shape[d];
+            idx[d] = r - q * shape[d];
+            soff += idx[d] * p.strides[d];
+            r = q;
+        }
+        idx[0] = r;
+        soff += r * p.strides[0];
+        const bool full = at + VE <= count;
+        u32x4 v = {0, 0, 0, 0};
+        if (p.strides[RANK - 1] == 1 && idx[RANK - 1] + VE <= shape[RANK - 1]) {
+            v = perm_detail::load128u<false>(src + soff * W);
+        } else {
+#pragma unroll
+            for (uint32_t e = 0; e < VE; ++e) {
+                if (at + e < count) {
+#pragma unroll
+                    for (int w = 0; w < W; ++w) v[e * W + w] = src[soff * W + w];
+                }
+                // The next element: a carry runs up through the axes that end here.
+                bool carry = true;
+#pragma unroll
+                for (int d = RANK - 1; d >= 0; --d) {
+                    if (carry) {
+                        soff += p.strides[d];
+                        carry = ++idx[d] == shape[d];
+                        if (carry) {
+                            soff -= static_cast<int64_t>(shape[d]) * p.strides[d];
+                            idx[d] = 0;
+                        }
+                    }
+                }
+            }
+        }
+        if constexpr (CONJ) {
+#pragma unroll
+            for (uint32_t e = 0; e < VE; ++e) v[e * W + 1] ^= SIGN;
+        }
+        uint32_t* q = dst + at * W;
+        if (full) {
+            perm_detail::store128u<false>(q, v);
+        } else {
+#pragma unroll
+            for (uint32_t e = 0; e < VE; ++e)
+                if (at + e < count)
+                    for (int w = 0; w < W; ++w) q[e * W + w] = v[e * W + w];
+        }
+    }
+}
+
 constexpr uint64_t TILE_GRID_CAP = 1u << 22;
 constexpr uint64_t COPY_GRID_CAP = 1u << 20;
 
@@ -92,6 +162,14 @@ template <int W, bool CONJ, bool NT>
 void copy_t(hipStream_t s, const PermCopyArgs& a) {
     const dim3 grid(static_cast<uint32_t>(perm_copy_workgroups(a.count, W)));
     hipLaunchKernelGGL((perm_copy<W, CONJ, NT>), grid, dim3(PERM_THREADS), 0, s, a);
+}
+
+template <int W, bool CONJ>
+void rows_t(hipStream_t s, const PermCopyArgs& a) {
+    const dim3 grid(static_cast<uint32_t>(perm_copy_workgroups(a.count, W)));
+    if (a.rank == 2) hipLaunchKernelGGL((perm_rows<W, CONJ, 2>), grid, dim3(PERM_THREADS), 0, s, a);
+    else if (a.rank == 3) hipLaunchKernelGGL((perm_rows<W, CONJ, 3>), grid, dim3(PERM_THREADS), 0, s, a);
+    else hipLaunchKernelGGL((perm_rows<W, CONJ, 4>), grid, dim3(PERM_THREADS), 0, s, a);
 }
 
 }  // namespace
@@ -130,7 +208,11 @@ void launch_perm_tile(Context* ctx, hipStream_t s, const PermTileArgs& a, int wo
 void launch_perm_copy(Context* ctx, hipStream_t s, const PermCopyArgs& a, int words, bool conj) {
     const bool nt = a.streaming != 0;
     const char* name;
-    if (words == 1) {
+    if (a.contiguous == 0 && a.rank >= 2 && a.rank <= 4 && a.count < (1ull << 32)) {
+        if (words == 1) rows_t<1, false>(s, a), name = "perm_rows_w1";
+        else if (!conj) rows_t<2, false>(s, a), name = "perm_rows_w2";
+        else rows_t<2, true>(s, a), name = "perm_rows_conj_w2";
+    } else if (words == 1) {
         if (nt) copy_t<1, false, true>(s, a), name = "perm_copy_w1_stream";
         else copy_t<1, false, false>(s, a), name = "perm_copy_w1";
     } else if (!conj) {

@@ -29,6 +29,18 @@ constexpr uint32_t SIGN = 0x80000000u;
 
 // 128-bit global accesses; NT marks them non-temporal (streamed past the caches).
 // Tile kernels take NTM: bit 0 makes the loads non-temporal, bit 1 the stores.
+// The same of words that are only known to be 4-byte aligned (a global access needs no more).
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool NT>
+__device__ inline u32x4 load128u(const uint32_t* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4u*>(p));
+    else return *reinterpret_cast<const u32x4u*>(p);
+}
+template <bool NT>
+__device__ inline void store128u(uint32_t* p, u32x4 v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4u*>(p));
+    else *reinterpret_cast<u32x4u*>(p) = v;
+}
 template <bool NT>
 __device__ inline u32x4 load128(const uint32_t* p) {
     if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
@@ -64,9 +76,9 @@ __global__ __launch_bounds__(NTH) void perm_tile(PermTileArgs p) {
         // (rows off the 128-byte grid) meet in one L2 instead of each moving a part of it.
         // Measured, us: 8191 x 4099 85 -> 65, 8188 x 4100 86 -> 60, 2476 x 3864 16.8 -> 13.2, rows on the grid 4096^2
         // 30.5 -> 29.3. Streaming tiles write whole lines past the L2 and keep the plain order (8192 x 4096
-        // 48.6 against 49.5).
+        // 48.6 against 49.5), and so do planes of one tile (5005 of 33 x 7: 21.3 against 22.4).
         uint64_t t = lin;
-        if constexpr (NTM == 0) {
+        if (NTM == 0 && per_outer > 1) {
             const uint64_t q8 = p.total_tiles >> 3, r8 = p.total_tiles & 7u, xcd = lin & 7u;
             t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (lin >> 3);
         }
