@@ -425,7 +425,8 @@ int load_mode_half(uintptr_t base, uint64_t off, uint64_t sb, uint64_t srow, uin
 // the f32 matrix instruction for short chunks (us, f32 against pieces): split 128 deep 13.6 against
 // 14.0 (200 x 190 x 2000), 512 deep 51 against 35 (1984 x 128 x 4928); operands with aligned unit-stride axes 336 deep 31
 // against 31 (17 x 880 x 176), 1008 deep 90 against 81 (12 x 896 x 368); and whole K over four
-// wave groups with A along K 28.8 against 29.5 (1024 x 1024 x 1000), A along M 40 against 30.
+// wave groups with A along K 28.8 against 29.5 (1024 x 1024 x 1000), A along M 40 against 30. Full 64x64 tiles on
+// gemm_f32_kw gain too little to move (256 x 256 x 65536 77.0 against 75.7).
 bool pieces_fit(const GemmArgs& t, int a_mode, int b_mode) {
     if (t.kernel != KERN_TILE && t.kernel != KERN_DIRECT && t.kernel != KERN_PIPE && t.kernel != KERN_SK) return false;
     if (t.tile < GEMM_SMALL_TILE || (t.tile != PIPE_TALL_M && t.tile_n < t.tile)) return false;
@@ -434,7 +435,7 @@ bool pieces_fit(const GemmArgs& t, int a_mode, int b_mode) {
     if (t.tile == GEMM_SMALL_TILE) {
         const bool aligned = a_mode != LOAD_S && b_mode != LOAD_S;
         if (t.k_chunk < (aligned ? 512u : 256u)) return false;
-        if (t.kernel == KERN_DIRECT && a_mode == LOAD_K) return false;
+        if (t.kernel == KERN_PIPE || (t.kernel == KERN_DIRECT && a_mode == LOAD_K)) return false;
     }
     auto near = [](uint64_t rows, int64_t srow, int64_t sk) {
         const uint64_t limit = 1ull << 29;  // elements, half of 2^32 bytes

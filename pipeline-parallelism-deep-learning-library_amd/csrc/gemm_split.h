@@ -175,14 +175,16 @@ struct B3Loader {
     }
     __device__ __forceinline__ void advance(int slices = 1) { base += slices * B3_BK * sk; }
 
-    // Row i of the block: its pieces into a stage.
-    template <bool SCALE>
+    // Row i of the block: its pieces into a stage. NEG: of the negated elements (a source modifier of
+    // the conversion's first instructions).
+    template <bool SCALE, bool NEG = false>
     __device__ __forceinline__ void store_row(char* stage, const B3Block& x, int i, float scale, B3Low& low) const {
         float e[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             e[j] = MODE == LOAD_MN ? x.v[j][i] : x.v[i][j];
             if constexpr (SCALE) e[j] = scale * e[j];
+            if constexpr (NEG) e[j] = -e[j];
         }
         uint32_t lo[3], hi[3];
         b3_split(e[0], e[1], lo, low);
@@ -229,7 +231,7 @@ __device__ __forceinline__ void b3_block(const bf16x8 (&a)[3], const bf16x8 (&b)
 // whether some element was too small for its pieces.
 template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
 __device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const float* A, const float* B,
-                                        uint32_t m0, uint32_t n0, uint32_t klen, floatx16 (&acc)[FM][FN]) {
+                                        uint32_t m0, uint32_t n0, uint32_t klen, float sign, floatx16 (&acc)[FM][FN]) {
     constexpr int RA = 32 * FM * WM, RB = 32 * FN * WN;
     using GA = B3Geo<RA>;
     using GB = B3Geo<RB>;
@@ -375,11 +377,11 @@ __device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const flo
     if (wave < WA) {
         B3Loader<AM, RA, EDGE> ld;
         ld.init(A, p.a_sm, p.a_sk, m0, p.m, tid);
-        with(&ld, p.scale_b ? 1.0f : p.alpha, smem);
+        with(&ld, p.scale_b ? 1.0f : sign * p.alpha, smem);
     } else if (wave < WA + WB) {
         B3Loader<BMD, RB, EDGE> ld;
         ld.init(B, p.b_sn, p.b_sk, n0, p.n, tid - RA);
-        with(&ld, p.scale_b ? p.alpha : 1.0f, smem + GA::BYTES);
+        with(&ld, p.scale_b ? sign * p.alpha : 1.0f, smem + GA::BYTES);
     } else {
         void* none = nullptr;
         loop(&none, std::false_type{}, 1.0f, smem);
@@ -414,11 +416,21 @@ __device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const
     }
 }
 
-// A tile's sums over k [0, klen), by whichever way holds its elements.
+// A tile's sums over k [0, klen), by whichever way holds its elements. The bf16 instruction cuts the
+// bits that its accumulator has no room for, so a sum is a little low (2e-7 of it at K = 4096); `negative`
+// sums the negated products and negates the sum, which is then a little high: every other split of K does, and the
+// splits' errors cancel instead of adding up.
 template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
 __device__ __forceinline__ void b3_sums(const GemmArgs& p, char* smem, const float* A, const float* B, uint32_t m0,
-                                        uint32_t n0, uint32_t klen, int wave, int lane, floatx16 (&acc)[FM][FN]) {
-    const bool bad = b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, acc);
+                                        uint32_t n0, uint32_t klen, bool negative, int wave, int lane,
+                                        floatx16 (&acc)[FM][FN]) {
+    const bool bad = b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, negative ? -1.0f : 1.0f, acc);
+    if (negative) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = -acc[i][j];
+    }
     // x * 0 is 0 unless x is infinite or NaN. Rows and columns past the output's edge hold
     // whatever the stages held, and do not count.
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
@@ -467,7 +479,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
     const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
     floatx16 acc[FM][FN];
     b3_zero(acc);
-    b3_sums<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, wave, lane, acc);
+    b3_sums<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, split & 1u, wave, lane, acc);
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
     float* C = p.partial != nullptr ? p.partial + static_cast<int64_t>(plane) * p.m * p.n
                                     : p.c + static_cast<int64_t>(bi) * p.c_sb;
@@ -500,7 +512,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
 // share a compute unit. The sums meet in LDS as (s0 + s1) + (s2 + s3), each wave storing one block. Bound:
 // the VALU, at 110-115 TFLOP/s. Against the f32 instruction: 3001 x 2011 x 1537 with odd rows 459 -> 164 us
 // (32-bit loads before), 2300 x 2304 x 2304 274 -> 219, 320 x 352 x 97536 418 -> 224, 37^6 in rank 4 147 -> 56,
-// 256 x 256 x 65536 77.4 -> 75.5.
+// 1000 x 1024 x 1024 with A along M 40 -> 30.
 template <int AM, int BMD, bool EDGE>
 __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     constexpr int R = 64, W = 4;
@@ -538,8 +550,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     floatx16 acc[2][2];
     b3_zero(acc);
     B3Low low;
-    auto loop = [&](auto scaled) __attribute__((always_inline)) {
-        constexpr bool SCALE = decltype(scaled)::value;
+    // Waves 1 and 3 sum the negated products: see b3_sums.
+    auto loop = [&](auto scaled, auto negated) __attribute__((always_inline)) {
+        constexpr bool SCALE = decltype(scaled)::value, NEG = decltype(negated)::value;
         B3Block xa[2], xb[2];
         auto fetch = [&](uint32_t s, int to) __attribute__((always_inline)) {
             if (s != 0 && s < slices) {
@@ -557,7 +570,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
         auto put = [&](int from) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                la.template store_row<SCALE>(mine, xa[from], r, alpha_a, low);
+                la.template store_row<SCALE, NEG>(mine, xa[from], r, alpha_a, low);
                 lb.template store_row<SCALE>(mine + G::BYTES, xb[from], r, alpha_b, low);
             }
         };
@@ -599,8 +612,13 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
         }
         if (s < slices) step(std::integral_constant<int, 0>{}, s);
     };
-    if (p.alpha != 1.0f) loop(std::true_type{});
-    else loop(std::false_type{});
+    if (p.alpha != 1.0f) {
+        if (wave & 1) loop(std::true_type{}, std::true_type{});
+        else loop(std::true_type{}, std::false_type{});
+    } else {
+        if (wave & 1) loop(std::false_type{}, std::true_type{});
+        else loop(std::false_type{}, std::false_type{});
+    }
 
     const bool tiny = __syncthreads_or(low.tiny());
     {
@@ -610,7 +628,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) q[((i * 2 + j) * 16 + r) * 64] = acc[i][j][r];
+                for (int r = 0; r < 16; ++r) q[((i * 2 + j) * 16 + r) * 64] = (wave & 1) ? -acc[i][j][r] : acc[i][j][r];
     }
     __syncthreads();
     const int bm = wave >> 1, bn = wave & 1;
@@ -684,7 +702,7 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_b3sk(GemmArgs p) {
         const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
         floatx16 acc[FM][FN];
         b3_zero(acc);
-        b3_sums<AM, BMD, 2, 2, FM, FN, false>(p, smem, A, B, m0, n0, len * STEP, wave, lane, acc);
+        b3_sums<AM, BMD, 2, 2, FM, FN, false>(p, smem, A, B, m0, n0, len * STEP, false, wave, lane, acc);
         if (whole) {
             pl_store_c<FN>(p, acc, bi, m0, n0);
         } else {
