@@ -8,7 +8,8 @@ line carries the permutation headline (GB/s on the 1 GiB-traffic [512,1024,256] 
 materialization) and a [value, unit, roofline frac] summary of every benchmark configuration;
 each workload's full record (plan, kernels, median/best, CPU baselines) goes to the --detail
 file. Rooflines:
-  contraction: achieved = 2*B*M*N*K / mean kernel time, peak = 157.3 TFLOP/s fp32 MFMA
+  contraction: achieved = 2*B*M*N*K / mean kernel time, peak = 157.3 TFLOP/s fp32 MFMA, or
+               2500 / 6 where an f32 product is six bf16 ones (the gemm_f32_b3 kernels)
   permutation: achieved = 2*numel*4 B / mean kernel time,  peak = 8000 GB/s HBM
 Kernel time is measured with HIP events recorded on the stream the kernels are launched on,
 around `steps` back-to-back launches after `warmup` untimed ones (and at least `--warmup-ms`
@@ -36,11 +37,20 @@ sys.path.insert(0, str(REPO))
 
 METRIC = "contraction TFLOP/s (% fp32 MFMA peak); permute GB/s (% HBM peak)"
 PEAK_TFLOPS = 157.3     # MI355X dense fp32 MFMA
+PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 PEAK_GBS = 8000.0       # MI355X HBM3E
 PEAK_F64_TFLOPS = 78.6  # MI355X dense fp64 MFMA
-# MI355X published fp32 vector peak. The 16-bit Backend gemm spends two f32 operations (one
-# multiply, one add, never fused) per term; it is priced against this figure.
+# MI355X published fp32 vector peak, and its fp32 MFMA peak. The 16-bit Backend gemm spends two f32
+# operations (a multiply and an add, or one fused on the matrix cores) per term.
 PEAK_VECTOR_TFLOPS = 157.3
+
+
+def mfma_peak(kernels):
+    """TFLOP/s of f32 product that the matrix instruction of these kernels could reach: the
+    three-piece kernels (gemm_f32_b3*) spend six bf16 products on each f32 one."""
+    if any(k.startswith("gemm_f32_b3") for k in kernels):
+        return round(PEAK_BF16_TFLOPS / 6, 1)
+    return PEAK_TFLOPS
 
 
 class HipEvents:
@@ -245,7 +255,7 @@ def bench_gemm(ctx, events, pool, L, C, name, m, n, k, args, a_t=False, b_t=Fals
             extra = {"ms_graph": g, "tflops_graph": flops / (g * 1e-3) / 1e12}
     return {"name": name, "ms": ms, "ms_median": med, "ms_best": best,
             "host_ms": HOST_MS[launch], "tflops": tflops, **extra,
-            "frac": tflops / PEAK_TFLOPS,
+            "peak": mfma_peak(kernels), "frac": tflops / mfma_peak(kernels),
             "plan": {k_: plan[k_] for k_ in ("kind", "kernel", "tile", "a_mode", "b_mode",
                                               "splits", "workgroups")},
             "kernels": kernels, "_host": (a, b), "_geom": (m, n, k, a_t, b_t, batch, beta)}
@@ -321,9 +331,10 @@ def bench_contract(ctx, events, pool, L, C, name, a_spec, b_spec, c_spec, args, 
         if g:
             extra = {"ms_graph": g, "tflops_graph": flops / (g * 1e-3) / 1e12,
                      "gbs_graph": nbytes / (g * 1e-3) / 1e9}
-    mfma_bound = flops / (PEAK_TFLOPS * 1e12) >= nbytes / (PEAK_GBS * 1e9)
-    roof = ({"bound": "mfma", "achieved": tflops, "peak": PEAK_TFLOPS, "unit": "TFLOP/s",
-             "frac": tflops / PEAK_TFLOPS} if mfma_bound else
+    peak = mfma_peak(kernels)
+    mfma_bound = flops / (peak * 1e12) >= nbytes / (PEAK_GBS * 1e9)
+    roof = ({"bound": "mfma", "achieved": tflops, "peak": peak, "unit": "TFLOP/s",
+             "frac": tflops / peak} if mfma_bound else
             {"bound": "hbm", "achieved": gbs, "peak": PEAK_GBS, "unit": "GB/s",
              "frac": gbs / PEAK_GBS})
     return {"name": name, "ms": ms, "ms_median": med, "ms_best": best, "host_ms": HOST_MS[launch],
@@ -439,10 +450,9 @@ def bench_gemm_f16(ctx, events, pool, L, C, m, n, k, args):
 
 
 def bench_backend_gemm16(events, args, timed_fn, m=4096, n=4096, k=4096):
-    """Backend::gemm on F16 tensors, bit-exact with CpuBackend (one lane per output runs the
-    reference's serial f32 chain): 10^12 terms (multiply-add pairs) per second, and the two f32
-    operations per term against the published 157.3 TFLOP/s fp32 vector peak (which counts
-    packed FMA; the chain can use neither packing nor fusion)."""
+    """Backend::gemm on F16 tensors, bit-exact with CpuBackend (each output is the reference's
+    serial f32 chain, on the f32 matrix cores): 10^12 terms (multiply-add pairs) per second, and the
+    two f32 operations per term against 157.3 TFLOP/s."""
     import oracle
     from linalg_hip import backend as B
     hb = B.HipBackend(0)
@@ -456,7 +466,7 @@ def bench_backend_gemm16(events, args, timed_fn, m=4096, n=4096, k=4096):
     terms = m * n * k / (ms * 1e-3) / 1e12
     res = {"name": f"Backend::gemm f16 {m}x{n}x{k} (CpuBackend's f32 chain, bit-exact)", "ms": ms,
            "tterms": terms, "tflops_vector": 2 * terms, "frac_vector": 2 * terms / PEAK_VECTOR_TFLOPS,
-           "kernel": "gemm16_seq<0, 8>"}
+           "kernel": "gemm16_chain<0, 4, true, false>"}
     hb.close()
     if not args.no_cpu:
         rows = 4
@@ -798,7 +808,7 @@ def headline_line(results, args, train, bgemm16, detail_path):
                        "m": 4096, "n": 4096, "k": 4096, "parallelism": "single-gpu"}}
     if head:
         line["roofline"] = {"bound": "mfma", "achieved": round(head["tflops"], 3),
-                            "peak": PEAK_TFLOPS, "unit": "TFLOP/s",
+                            "peak": head.get("peak", PEAK_TFLOPS), "unit": "TFLOP/s",
                             "frac": round(head["frac"], 4),
                             "traffic": traffic_from_profile("gemm4096"),
                             "kernel": ", ".join(head.get("kernels", [])),
@@ -947,7 +957,7 @@ def main() -> int:
         ms = y["ms"] + dx["ms"] + dw["ms"]
         tf = 3 * 2.0 * M * N * K / (ms * 1e-3) / 1e12
         return {"name": "C5 linear-layer step (3 gemms)", "ms": ms, "tflops": tf,
-                "frac": tf / PEAK_TFLOPS, "parts": [y, dx, dw]}
+                "frac": tf / max(r["peak"] for r in (y, dx, dw)), "parts": [y, dx, dw]}
     run("c5", c5)
     run("c2a", lambda: bench_perm(ctx, events, pool, L, P, "C2a [64,128,64,32] perm (0,2,3,1)",
                                   [64, 128, 64, 32], [0, 2, 3, 1], 3, args))

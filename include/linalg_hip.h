@@ -272,8 +272,9 @@ typedef struct lg_tensor {
  * `accumulate`, :664-691): per output, acc = beta*C in f32 (0 when beta is 0), then
  * acc = acc + (alpha*a)*b in k order, every multiply and add rounded to f32, stored rounded
  * to the 16-bit type to nearest even (the half crate's from_f32_const); only NaN payloads may
- * differ. This runs on the vector ALUs (one lane per output), not the matrix cores, whose
- * summation order is their own. The checks run before `ctx` is used.
+ * differ. Where (alpha*a)*b needs no rounding (alpha of at most 2 significant bits for F16, 8
+ * for BF16) the chain runs on the f32 matrix cores, which add products in k order; otherwise
+ * on the vector ALUs, one lane per output. The checks run before `ctx` is used.
  * Enqueues on `stream` (NULL = context stream) and returns before the device finishes, as
  * the GPU backends do (crates/core/src/lib.rs:72-82). On any error nothing is launched. */
 lg_core_error lg_backend_gemm(lg_ctx* ctx, void* stream, const lg_tensor* a, const lg_tensor* b,
