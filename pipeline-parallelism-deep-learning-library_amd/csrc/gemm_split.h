@@ -204,6 +204,15 @@ __device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const
                                                   uint32_t n0, uint32_t klen, int wave, int lane,
                                                   floatx16 (&acc)[FM][FN]);
 
+// Every LDS access of this wave done, then the workgroup's barrier. Waves that load nothing store
+// nothing either, and only the fences tell the compiler that what they read there changes.
+__device__ __forceinline__ void b3_barrier() {
+    __asm__ volatile("" ::: "memory");
+    wait_lgkm0();
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+}
+
 template <int FM, int FN>
 __device__ __forceinline__ void b3_zero(floatx16 (&acc)[FM][FN]) {
 #pragma unroll
@@ -308,8 +317,7 @@ __device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const flo
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            wait_lgkm0();
-            __builtin_amdgcn_s_barrier();
+            b3_barrier();
             constexpr int L = (FM - 1) & 1;
 #pragma unroll
             for (int r = 0; r < EARLY; ++r) put_row(r, P, x[X2]);
@@ -345,8 +353,7 @@ __device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const flo
 #pragma unroll
         for (int r = 0; r < EARLY; ++r) put_row(r, 1, x[1]);
         fetch(NX, x[0]);
-        wait_lgkm0();
-        __builtin_amdgcn_s_barrier();
+        b3_barrier();
         read_a(a[0], 0, 0);
         read_b(2, 0);
         read_b(1, 0);

@@ -74,11 +74,12 @@ __global__ __launch_bounds__(NTH) void perm_tile(PermTileArgs p) {
         // Cached tiles: workgroups are dealt to the eight XCDs in turn, and each XCD takes one
         // contiguous run of tiles, so that the tiles on either side of a line that no tile boundary falls on
         // (rows off the 128-byte grid) meet in one L2 instead of each moving a part of it.
-        // Measured, us: 8191 x 4099 85 -> 65, 8188 x 4100 86 -> 60, 2476 x 3864 16.8 -> 13.2, rows on the grid 4096^2
-        // 30.5 -> 29.3. Streaming tiles write whole lines past the L2 and keep the plain order (8192 x 4096
-        // 48.6 against 49.5), and so do planes of one tile (5005 of 33 x 7: 21.3 against 22.4).
+        // Measured, us: 8191 x 4099 85 -> 65, 8188 x 4100 86 -> 60, 2476 x 3864 16.8 -> 13.2. Rows on the grid keep
+        // the plain order ([64,2048,128] 21.5 against 25.2), and so do streaming tiles (8192 x 4096
+        // 48.6 against 49.5) and planes of one tile (5005 of 33 x 7: 21.3 against 22.4).
         uint64_t t = lin;
-        if (NTM == 0 && per_outer > 1) {
+        const bool off_grid = (p.src_sb * W) % 32 != 0 || (p.dst_sa * W) % 32 != 0;
+        if (NTM == 0 && per_outer > 1 && off_grid) {
             const uint64_t q8 = p.total_tiles >> 3, r8 = p.total_tiles & 7u, xcd = lin & 7u;
             t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (lin >> 3);
         }
