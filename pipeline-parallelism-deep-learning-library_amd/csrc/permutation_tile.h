@@ -76,7 +76,7 @@ __global__ __launch_bounds__(NTH) void perm_tile(PermTileArgs p) {
         // (rows off the 128-byte grid) meet in one L2 instead of each moving a part of it.
         // Measured, us: 8191 x 4099 85 -> 65, 8188 x 4100 86 -> 60, 2476 x 3864 16.8 -> 13.2. Rows on the grid keep
         // the plain order ([64,2048,128] 21.5 against 25.2), and so do streaming tiles (8192 x 4096
-        // 48.6 against 49.5) and planes of one tile (5005 of 33 x 7: 21.3 against 22.4).
+        // 48.6 against 49.5); a plane of one tile has no neighbour to meet.
         uint64_t t = lin;
         const bool off_grid = (p.src_sb * W) % 32 != 0 || (p.dst_sa * W) % 32 != 0;
         if (NTM == 0 && per_outer > 1 && off_grid) {
