@@ -430,7 +430,7 @@ int load_mode_half(uintptr_t base, uint64_t off, uint64_t sb, uint64_t srow, uin
 bool pieces_fit(const GemmArgs& t, int a_mode, int b_mode) {
     if (t.kernel != KERN_TILE && t.kernel != KERN_DIRECT && t.kernel != KERN_PIPE && t.kernel != KERN_SK) return false;
     if (t.tile < GEMM_SMALL_TILE || (t.tile != PIPE_TALL_M && t.tile_n < t.tile)) return false;
-        const uint32_t last = t.k - (t.splits - 1) * t.k_chunk;
+    const uint32_t last = t.k - (t.splits - 1) * t.k_chunk;
     if (std::min(t.k_chunk, last) < PIECES_MIN_K || t.m < 4 || t.n < 4) return false;
     if (t.tile == GEMM_SMALL_TILE) {
         const bool aligned = a_mode != LOAD_S && b_mode != LOAD_S;

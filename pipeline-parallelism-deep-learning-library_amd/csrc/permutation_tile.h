@@ -29,6 +29,16 @@ constexpr uint32_t SIGN = 0x80000000u;
 
 // 128-bit global accesses; NT marks them non-temporal (streamed past the caches).
 // Tile kernels take NTM: bit 0 makes the loads non-temporal, bit 1 the stores.
+template <bool NT>
+__device__ inline u32x4 load128(const uint32_t* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    else return *reinterpret_cast<const u32x4*>(p);
+}
+template <bool NT>
+__device__ inline void store128(uint32_t* p, u32x4 v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+    else *reinterpret_cast<u32x4*>(p) = v;
+}
 // The same of words that are only known to be 4-byte aligned (a global access needs no more).
 typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 template <bool NT>
@@ -40,16 +50,6 @@ template <bool NT>
 __device__ inline void store128u(uint32_t* p, u32x4 v) {
     if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4u*>(p));
     else *reinterpret_cast<u32x4u*>(p) = v;
-}
-template <bool NT>
-__device__ inline u32x4 load128(const uint32_t* p) {
-    if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-    else return *reinterpret_cast<const u32x4*>(p);
-}
-template <bool NT>
-__device__ inline void store128(uint32_t* p, u32x4 v) {
-    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
-    else *reinterpret_cast<u32x4*>(p) = v;
 }
 
 template <int W, bool CONJ, bool VEC, int TA, int TB, int NTM, int NTH>
