@@ -123,3 +123,19 @@ def test_elements_outside_the_pieces(ctx, pool, what, shape):
         assert np.array_equal(want[~fine & ~np.isnan(want)], got[~fine & ~np.isnan(want)])
         bound = (k + 2) * U * (np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64)))
     assert np.all(np.abs(got[fine] - want[fine]) <= bound[fine] + 1e-44)
+
+
+@pytest.mark.parametrize("shape", [(2045, 1930, 77), (1000, 1020, 1537), (2304, 2304, 256)])
+@pytest.mark.parametrize("exponent", [-58, -64, -70, -74])
+def test_products_below_the_normal_range(ctx, pool, shape, exponent):
+    """Products of the later pieces, or all of them, are subnormal in f32: each of the up to 6 K sums
+    may lose half of a least subnormal, and no more."""
+    m, n, k = shape
+    g = rng(9400)
+    a = np.ldexp(g.standard_normal((m, k)), exponent).astype(np.float32)
+    b = np.ldexp(g.standard_normal((k, n)), exponent).astype(np.float32)
+    got, name = _product(ctx, pool, a, b, m == 1000, False)
+    assert name.startswith("gemm_f32_b3"), name
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    bound = (k + 2) * U * (np.abs(a64) @ np.abs(b64)) + 6 * k * 2.0 ** -149
+    assert np.all(np.abs(got - a64 @ b64) <= bound), float(np.max(np.abs(got - a64 @ b64) / bound))
