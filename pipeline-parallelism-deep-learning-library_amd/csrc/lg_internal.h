@@ -353,6 +353,7 @@ struct PermTileArgs {
     uint32_t outer_shape[PERM_MAX_RANK];
     int64_t outer_src[PERM_MAX_RANK];
     int64_t outer_dst[PERM_MAX_RANK];
+    uint32_t order;  // walk over the tiles, set at the launch (perm_tile_order)
 };
 
 struct PermCopyArgs {

@@ -184,8 +184,28 @@ uint64_t perm_copy_workgroups(uint64_t count, int words) {
     return g < COPY_GRID_CAP ? (g ? g : 1) : COPY_GRID_CAP;
 }
 
-void launch_perm_tile(Context* ctx, hipStream_t s, const PermTileArgs& a, int words, bool conj,
+// The walk over a cached view's tiles. 0: (outer, ta, tb), tb fastest. 1: workgroups are dealt to the eight
+// XCDs in turn, and each XCD takes one contiguous run of that order, so that the tiles on either side of a
+// destination line that no tile boundary falls on (rows off the 128-byte grid) meet in one L2 instead of each
+// writing a part of it. 2: runs with ta fastest, where few tiles along a would give whole XCDs the last,
+// partly filled ones. Measured, us: 8191 x 4099 85 -> 65 (77 by order 2, so the limit), 2476 x 3864 16.8 -> 13.2,
+// 4855 x 1187 13.1 -> 10.8 (11.8 by order 1; 7900 x 129 5.0 against 4.3). Runs lose where no destination line is
+// cut: rows on the grid (77088 x 229 35.0 against 41.4), one tile per row ([28,1372,240] by 1,2,0 16.7
+// against 18.8), streaming tiles (8192 x 4096 48.6 against 49.5); and on aligned rows of many planes
+// ([100,180,16,36] by 2,0,3,1 22.9 against 24.6; unaligned [66,30,47,8] by 3,1,2,0 gains, 15.6 -> 12.9).
+uint32_t perm_tile_order(const PermTileArgs& a, int words, bool vec, bool streaming) {
+    constexpr uint32_t FEW = 32;
+    if (streaming || a.tiles_b < 2 || (a.dst_sa * words) % 32 == 0 || (vec && a.outer_rank != 0) ||
+        a.total_tiles > 0xffffffffull) {
+        return 0;
+    }
+    return a.outer_rank == 0 && a.tiles_b > a.tiles_a && a.tiles_a <= FEW ? 2 : 1;
+}
+
+void launch_perm_tile(Context* ctx, hipStream_t s, const PermTileArgs& args, int words, bool conj,
                       bool vec, bool streaming) {
+    PermTileArgs a = args;
+    a.order = perm_tile_order(a, words, vec, streaming);
     constexpr int TS = PERM_STREAM_TILE_A, TN = PERM_TILE_A;
     const char* name = nullptr;
     if (words == 1) {

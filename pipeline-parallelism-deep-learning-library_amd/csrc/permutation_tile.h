@@ -7,8 +7,8 @@
 // b (destination unit stride). A TA x TB element tile is read with 128-bit loads running along
 // a, staged in LDS with an odd word pitch (TA*W + 1) so both the row-wise fill and the
 // column-wise drain spread over the banks, and written with 128-bit stores running along b.
-// Tiles are walked with a grid stride in the order (outer, ta, tb), tb fastest (cached tiles: each
-// XCD in a run of its own): concurrently
+// Tiles are walked with a grid stride in the order (outer, ta, tb), tb fastest (or in a run per
+// XCD, perm_tile_order): concurrently
 // running workgroups write consecutive TB-element segments of the same TA destination rows, so
 // every destination row is written front to back, and read consecutive bands of source rows.
 // (On a 1 GiB transpose this order measured 2-3% faster than ta fastest on MI355X.)
@@ -71,30 +71,42 @@ __global__ __launch_bounds__(NTH) void perm_tile(PermTileArgs p) {
     const uint64_t per_outer = static_cast<uint64_t>(p.tiles_a) * p.tiles_b;
 
     for (uint64_t lin = blockIdx.x; lin < p.total_tiles; lin += gridDim.x) {
-        // Cached tiles: workgroups are dealt to the eight XCDs in turn, and each XCD takes one
-        // contiguous run of tiles, so that the tiles on either side of a line that no tile boundary falls on
-        // (rows off the 128-byte grid) meet in one L2 instead of each moving a part of it.
-        // Measured, us: 8191 x 4099 85 -> 65, 8188 x 4100 86 -> 60, 2476 x 3864 16.8 -> 13.2. Rows on the grid keep
-        // the plain order ([64,2048,128] 21.5 against 25.2), and so do streaming tiles (8192 x 4096
-        // 48.6 against 49.5); a plane of one tile has no neighbour to meet.
-        uint64_t t = lin;
-        const bool off_grid = (p.src_sb * W) % 32 != 0 || (p.dst_sa * W) % 32 != 0;
-        if (NTM == 0 && per_outer > 1 && off_grid) {
-            const uint64_t q8 = p.total_tiles >> 3, r8 = p.total_tiles & 7u, xcd = lin & 7u;
-            t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (lin >> 3);
-        }
-        uint64_t outer = t / per_outer;
-        const uint64_t rem = t - outer * per_outer;
-        const uint32_t ta = static_cast<uint32_t>(rem / p.tiles_b);
-        const uint32_t tb = static_cast<uint32_t>(rem - static_cast<uint64_t>(ta) * p.tiles_b);
         int64_t sbase = static_cast<int64_t>(p.src_offset);
         int64_t dbase = static_cast<int64_t>(p.dst_offset);
-        for (int d = static_cast<int>(p.outer_rank) - 1; d >= 0; --d) {
-            const uint64_t q = outer / p.outer_shape[d];
-            const int64_t c = static_cast<int64_t>(outer - q * p.outer_shape[d]);
-            sbase += c * p.outer_src[d];
-            dbase += c * p.outer_dst[d];
-            outer = q;
+        uint32_t ta, tb;
+        if (p.total_tiles <= 0xffffffffull) {
+            // 32-bit divisions; p.order: see perm_tile_order.
+            uint32_t t = static_cast<uint32_t>(lin);
+            if (NTM == 0 && p.order != 0) {
+                const uint32_t total = static_cast<uint32_t>(p.total_tiles), q8 = total >> 3, r8 = total & 7u, xcd = t & 7u;
+                t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (t >> 3);
+            }
+            const uint32_t per = static_cast<uint32_t>(per_outer);
+            uint32_t outer = 0, rem = t;
+            if (p.outer_rank != 0) outer = t / per, rem = t - outer * per;
+            const uint32_t fast = NTM == 0 && p.order == 2 ? p.tiles_a : p.tiles_b;
+            const uint32_t hi = rem / fast, lo = rem - hi * fast;
+            ta = NTM == 0 && p.order == 2 ? lo : hi;
+            tb = NTM == 0 && p.order == 2 ? hi : lo;
+            for (int d = static_cast<int>(p.outer_rank) - 1; d >= 0; --d) {
+                const uint32_t ext = static_cast<uint32_t>(p.outer_shape[d]), q = outer / ext;
+                const int64_t c = outer - q * ext;
+                sbase += c * p.outer_src[d];
+                dbase += c * p.outer_dst[d];
+                outer = q;
+            }
+        } else {
+            uint64_t outer = lin / per_outer;
+            const uint64_t rem = lin - outer * per_outer;
+            ta = static_cast<uint32_t>(rem / p.tiles_b);
+            tb = static_cast<uint32_t>(rem - static_cast<uint64_t>(ta) * p.tiles_b);
+            for (int d = static_cast<int>(p.outer_rank) - 1; d >= 0; --d) {
+                const uint64_t q = outer / p.outer_shape[d];
+                const int64_t c = static_cast<int64_t>(outer - q * p.outer_shape[d]);
+                sbase += c * p.outer_src[d];
+                dbase += c * p.outer_dst[d];
+                outer = q;
+            }
         }
         const uint32_t a0 = ta * TA, b0 = tb * TB;
         // Workgroup-uniform: the whole tile lies inside the view and 128-bit accesses are
