@@ -7,11 +7,12 @@
 // v_mfma_f32_32x32x16_bf16 adds sixteen of them into an f32 accumulator, so a sum over K is
 // rounded about 6 K / 16 times instead of the K times of v_mfma_f32_32x32x2_f32.
 //
-// The pieces cover f32's range down to 2^-110 or so, below which the last of them would need
-// bits that bf16 does not have, and up to bf16's largest value. A workgroup that meets a smaller
-// element, or whose sums come out as anything but finite numbers (an infinity or a NaN in an
-// operand or an overflow: x - x0 turns them into NaN), computes its tile again with the f32
-// matrix instruction on the operands themselves (b3_redo).
+// Elements are scaled by 2^23 before they are split and the sums by 2^-46 after: an f32, subnormals
+// included, is a whole multiple of 2^-149, so a scaled one is a whole multiple of 2^-126 and each of its pieces
+// zero or a normal bf16. So the pieces hold every element below 2^104 whole, whatever its size. A
+// workgroup whose scaled sums come out as anything but finite numbers (an infinity or a NaN in an operand,
+// an element of 2^104 or more, a sum of 2^82 or more: x - x0 turns an infinity into NaN) computes
+// its tile again with the f32 matrix instruction on the operands themselves (b3_redo).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,7 +27,6 @@ namespace gemm_detail {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef unsigned short ushortx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 // Four floats that are only known to be 4-byte aligned (global_load_dwordx4 needs no more).
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -47,33 +47,16 @@ struct B3Geo {
     static constexpr int BYTES = 3 * PL;
 };
 
-// Elements below 2^(B3_LEAST - 127) and not zero go to b3_redo. (From exponent 17 on all three
-// pieces of an f32 are exact; checked on every exponent and 2^21 elements each.)
-constexpr uint32_t B3_LEAST = 24;
+// The scale of the operands' elements, and that of the sums back (see the file's head). A test of the elements
+// instead, with the tile computed again where one is too small, cost as much per element and 4096^3 with
+// one element of 1e-35 4028 us, against 600 with the scale.
+constexpr float B3_UP = 0x1p23f, B3_DOWN = 0x1p-46f;
 
-// (x, y) -> three packed pairs of bf16 pieces. `low` keeps the least 2 |x0| - 1 (mod 2^16) seen,
-// in which zero counts as the largest. Thirteen VALU instructions a pair, four cycles each, and up to six of
-// them hide behind every MFMA. (v_dot2_f32_bf16 would do the subtraction and the unpacking in one, exactly,
-// but it does not run beside an MFMA: two of them cost an MFMA's time and a half.)
-struct B3Low {
-    ushortx2 v = {0xffff, 0xffff};
-    uint32_t two = 0x00020002u, ones = 0xffffffffu;
-    __device__ __forceinline__ B3Low() {
-        __asm__("" : "+s"(two));
-        __asm__("" : "+v"(ones));
-    }
-    __device__ __forceinline__ void see(uint32_t q) {
-        uint32_t d;
-        __asm__("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(d) : "v"(q), "s"(two), "v"(ones));
-        v = __builtin_elementwise_min(v, __builtin_bit_cast(ushortx2, d));
-    }
-    __device__ __forceinline__ bool tiny() const {
-        return min(static_cast<uint32_t>(v[0]), static_cast<uint32_t>(v[1])) < 2u * (B3_LEAST << 7) - 1u;
-    }
-};
-__device__ __forceinline__ void b3_split(float x, float y, uint32_t (&q)[3], B3Low& low) {
+// (x, y) -> three packed pairs of bf16 pieces. Eleven VALU instructions a pair and two for the scale, four
+// cycles each, and up to six of them hide behind every MFMA. (v_dot2_f32_bf16 would do the subtraction and the
+// unpacking in one, exactly, but it does not run beside an MFMA: two of them cost an MFMA's time and a half.)
+__device__ __forceinline__ void b3_split(float x, float y, uint32_t (&q)[3]) {
     q[0] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
-    low.see(q[0]);
     x = x - __builtin_bit_cast(float, q[0] << 16);
     y = y - __builtin_bit_cast(float, q[0] & 0xffff0000u);
     q[1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
@@ -90,14 +73,15 @@ struct B3Block {
 
 // Where a thread's block lies: byte offsets from the tile's first element of the slice, uniform strides,
 // and the LDS byte address of each of its rows (EDGE: rows past the operand's end are
-// the last ones again, and rows before the tile's first are not written).
+// the last ones again, and rows before the tile's first are written into their class's padding, which
+// nothing reads: a branch there would part the conversion from the MFMAs that hide it).
 template <int MODE, int R, bool EDGE>
 struct B3Loader {
     using G = B3Geo<R>;
     const float* base;  // the operand at the tile's first row (EDGE, LOAD_MN: see init) and current k
     int64_t srow, sk;
     uint32_t off[4];   // byte offset of load i (one offset and uniform strides unless EDGE)
-    uint32_t lds[4];   // byte address of row i in plane 0 (EDGE: 0xffffffff = not written)
+    uint32_t lds[4];   // byte address of row i in plane 0
     uint32_t k4;
 
     // p: the operand at (row 0 of the batch plane, first k). m0: the tile's first row, rows: the
@@ -130,7 +114,7 @@ struct B3Loader {
             if constexpr (MODE != LOAD_MN) off[i] += k4 * 4u * static_cast<uint32_t>(sk) * 4u;
             else off[i] += k4 * 4u * static_cast<uint32_t>(sk) * 4u;
             const uint32_t r = EDGE && MODE == LOAD_MN ? row0 + i - m0 : 4 * rq + i;
-            lds[i] = static_cast<int32_t>(r) < 0 ? 0xffffffffu : at + (r & 3u) * G::CLS + (r >> 2) * 16u;
+            lds[i] = at + (r & 3u) * G::CLS + (static_cast<int32_t>(r) < 0 ? R * 4u : (r >> 2) * 16u);
         }
     }
     __device__ __forceinline__ const float* at(int i) const {
@@ -175,25 +159,17 @@ struct B3Loader {
     }
     __device__ __forceinline__ void advance(int slices = 1) { base += slices * B3_BK * sk; }
 
-    // Row i of the block: its pieces into a stage. NEG: of the negated elements (a source modifier of
-    // the conversion's first instructions).
-    template <bool SCALE, bool NEG = false>
-    __device__ __forceinline__ void store_row(char* stage, const B3Block& x, int i, float scale, B3Low& low) const {
+    // Row i of the block: the pieces of its scaled elements into a stage.
+    __device__ __forceinline__ void store_row(char* stage, const B3Block& x, int i, float scale) const {
         float e[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            e[j] = MODE == LOAD_MN ? x.v[j][i] : x.v[i][j];
-            if constexpr (SCALE) e[j] = scale * e[j];
-            if constexpr (NEG) e[j] = -e[j];
-        }
+        for (int j = 0; j < 4; ++j) e[j] = scale * (MODE == LOAD_MN ? x.v[j][i] : x.v[i][j]);
         uint32_t lo[3], hi[3];
-        b3_split(e[0], e[1], lo, low);
-        b3_split(e[2], e[3], hi, low);
-        if (!(EDGE && MODE == LOAD_MN) || lds[i] != 0xffffffffu) {
-            char* q = EDGE && MODE == LOAD_MN ? stage + lds[i] : stage + lds[0] + i * G::CLS;
+        b3_split(e[0], e[1], lo);
+        b3_split(e[2], e[3], hi);
+        char* q = EDGE && MODE == LOAD_MN ? stage + lds[i] : stage + lds[0] + i * G::CLS;
 #pragma unroll
-            for (int s = 0; s < 3; ++s) *reinterpret_cast<uintx2*>(q + s * G::PL) = uintx2{lo[s], hi[s]};
-        }
+        for (int j = 0; j < 3; ++j) *reinterpret_cast<uintx2*>(q + j * G::PL) = uintx2{lo[j], hi[j]};
     }
 };
 
@@ -236,10 +212,10 @@ __device__ __forceinline__ void b3_block(const bf16x8 (&a)[3], const bf16x8 (&b)
     }
 }
 
-// One (32 FM WM) x (32 FN WN) tile over k [0, klen) from A and B (batch plane, first k): acc. Returns
-// whether some element was too small for its pieces.
+// One (32 FM WM) x (32 FN WN) tile over k [0, klen) from A and B (batch plane, first k): acc, of the scaled
+// elements, negated where `sign` is -1.
 template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
-__device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const float* A, const float* B,
+__device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const float* A, const float* B,
                                         uint32_t m0, uint32_t n0, uint32_t klen, float sign, floatx16 (&acc)[FM][FN]) {
     constexpr int RA = 32 * FM * WM, RB = 32 * FN * WN;
     using GA = B3Geo<RA>;
@@ -256,12 +232,10 @@ __device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const flo
     const uint32_t fa = fr * GA::CLS + fq + fh * GA::CH + wm * FM * 128;
     const uint32_t fb = fr * GB::CLS + fq + fh * GB::CH + wn * FN * 128 + GA::BYTES;
     const uint32_t full = klen / B3_BK, left = klen - full * B3_BK;
-    B3Low low;
 
-    auto loop = [&](auto* loader, auto scaled, float scale, char* mine) __attribute__((always_inline)) {
+    auto loop = [&](auto* loader, float scale, char* mine) __attribute__((always_inline)) {
         using LD = std::remove_pointer_t<decltype(loader)>;
         constexpr bool LOADS = !std::is_same_v<LD, void*>;
-        constexpr bool SCALE = decltype(scaled)::value;
         // Slice s passes through the registers x[s % NX] into stage s % 2. Step s multiplies slice s. All
         // of stage s % 2 is read and all of slice s + 1 written when the last row of blocks
         // begins: the step's one barrier stands there, and behind it, among that row's MFMAs, the
@@ -279,7 +253,7 @@ __device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const flo
             }
         };
         auto put_row = [&](int i, int stage, const B3Block& from) __attribute__((always_inline)) {
-            if constexpr (LOADS) loader->template store_row<SCALE>(mine + stage * ST, from, i, scale, low);
+            if constexpr (LOADS) loader->store_row(mine + stage * ST, from, i, scale);
         };
         bf16x8 a[2][3], b[FN][3];
         auto read_a = [&](bf16x8 (&to)[3], int i, int stage) __attribute__((always_inline)) {
@@ -377,23 +351,18 @@ __device__ __forceinline__ bool b3_tile(const GemmArgs& p, char* smem, const flo
             if (s < slices) step(std::integral_constant<int, 0>{}, s);
         }
     };
-    auto with = [&](auto* loader, float scale, char* mine) __attribute__((always_inline)) {
-        if (scale != 1.0f) loop(loader, std::true_type{}, scale, mine);
-        else loop(loader, std::false_type{}, scale, mine);
-    };
     if (wave < WA) {
         B3Loader<AM, RA, EDGE> ld;
         ld.init(A, p.a_sm, p.a_sk, m0, p.m, tid);
-        with(&ld, p.scale_b ? 1.0f : sign * p.alpha, smem);
+        loop(&ld, sign * (p.scale_b ? B3_UP : B3_UP * p.alpha), smem);
     } else if (wave < WA + WB) {
         B3Loader<BMD, RB, EDGE> ld;
         ld.init(B, p.b_sn, p.b_sk, n0, p.n, tid - RA);
-        with(&ld, p.scale_b ? sign * p.alpha : 1.0f, smem + GA::BYTES);
+        loop(&ld, p.scale_b ? B3_UP * p.alpha : B3_UP, smem + GA::BYTES);
     } else {
         void* none = nullptr;
-        loop(&none, std::false_type{}, 1.0f, smem);
+        loop(&none, 1.0f, smem);
     }
-    return low.tiny();
 }
 
 template <int FM, int FN, int WN>
@@ -431,13 +400,14 @@ template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
 __device__ __forceinline__ void b3_sums(const GemmArgs& p, char* smem, const float* A, const float* B, uint32_t m0,
                                         uint32_t n0, uint32_t klen, bool negative, int wave, int lane,
                                         floatx16 (&acc)[FM][FN]) {
-    const bool bad = b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, negative ? -1.0f : 1.0f, acc);
-    if (negative) {
+    b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, negative ? -1.0f : 1.0f, acc);
+    const float down = negative ? -B3_DOWN : B3_DOWN;
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) acc[i][j] = -acc[i][j];
-    }
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = down * acc[i][j][r];
     // x * 0 is 0 unless x is infinite or NaN. Rows and columns past the output's edge hold
     // whatever the stages held, and do not count.
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
@@ -454,7 +424,7 @@ __device__ __forceinline__ void b3_sums(const GemmArgs& p, char* smem, const flo
                     z = z + t;
                 }
             }
-    if (__syncthreads_or(bad || z != 0.0f)) b3_redo<FM, FN, WN>(p, A, B, m0, n0, klen, wave, lane, acc);
+    if (__syncthreads_or(z != 0.0f)) b3_redo<FM, FN, WN>(p, A, B, m0, n0, klen, wave, lane, acc);
 }
 
 // gemm_f32_b3<AM, BMD, WM, WN, FM, FN, EDGE>: C = beta * C + sum_k (alpha * a) * b, or raw split-K partials,
@@ -553,13 +523,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     lb.init(B, p.b_sn, p.b_sk, n0, p.n, lane);
     la.advance(wave);
     lb.advance(wave);
-    const float alpha_a = p.scale_b ? 1.0f : p.alpha, alpha_b = p.scale_b ? p.alpha : 1.0f;
+    // Waves 1 and 3 sum the negated products: see b3_sums.
+    const float scale_a = (wave & 1 ? -B3_UP : B3_UP) * (p.scale_b ? 1.0f : p.alpha);
+    const float scale_b = p.scale_b ? B3_UP * p.alpha : B3_UP, down = wave & 1 ? -B3_DOWN : B3_DOWN;
     floatx16 acc[2][2];
     b3_zero(acc);
-    B3Low low;
-    // Waves 1 and 3 sum the negated products: see b3_sums.
-    auto loop = [&](auto scaled, auto negated) __attribute__((always_inline)) {
-        constexpr bool SCALE = decltype(scaled)::value, NEG = decltype(negated)::value;
+    {
         B3Block xa[2], xb[2];
         auto fetch = [&](uint32_t s, int to) __attribute__((always_inline)) {
             if (s != 0 && s < slices) {
@@ -577,8 +546,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
         auto put = [&](int from) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                la.template store_row<SCALE, NEG>(mine, xa[from], r, alpha_a, low);
-                lb.template store_row<SCALE>(mine + G::BYTES, xb[from], r, alpha_b, low);
+                la.store_row(mine, xa[from], r, scale_a);
+                lb.store_row(mine + G::BYTES, xb[from], r, scale_b);
             }
         };
         // Other lanes read what a lane wrote: the compiler keeps their order, the LDS does by itself.
@@ -618,16 +587,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
             step(std::integral_constant<int, 1>{}, s + 1);
         }
         if (s < slices) step(std::integral_constant<int, 0>{}, s);
-    };
-    if (p.alpha != 1.0f) {
-        if (wave & 1) loop(std::true_type{}, std::true_type{});
-        else loop(std::true_type{}, std::false_type{});
-    } else {
-        if (wave & 1) loop(std::false_type{}, std::true_type{});
-        else loop(std::false_type{}, std::false_type{});
     }
 
-    const bool tiny = __syncthreads_or(low.tiny());
+    __syncthreads();  // the stages are free
     {
         float* q = reinterpret_cast<float*>(smem) + wave * (R * R) + lane;
 #pragma unroll
@@ -635,7 +597,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) q[((i * 2 + j) * 16 + r) * 64] = (wave & 1) ? -acc[i][j][r] : acc[i][j][r];
+                for (int r = 0; r < 16; ++r) q[((i * 2 + j) * 16 + r) * 64] = down * acc[i][j][r];
     }
     __syncthreads();
     const int bm = wave >> 1, bn = wave & 1;
@@ -651,7 +613,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
         if (!EDGE || (row_of(r) < p.m && col < p.n)) z = z + t;
     }
     // (Each wave's own block, over the whole chunk.)
-    if (__syncthreads_or(tiny || z != 0.0f)) b3_redo<1, 1, 2>(p, A, B, m0, n0, klen, wave, lane, v);
+    if (__syncthreads_or(z != 0.0f)) b3_redo<1, 1, 2>(p, A, B, m0, n0, klen, wave, lane, v);
     float* C = p.partial != nullptr ? p.partial + static_cast<int64_t>(plane) * p.m * p.n
                                     : p.c + static_cast<int64_t>(bi) * p.c_sb;
     const int64_t c_sm = p.partial != nullptr ? static_cast<int64_t>(p.n) : p.c_sm;

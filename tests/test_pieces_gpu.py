@@ -139,3 +139,28 @@ def test_products_below_the_normal_range(ctx, pool, shape, exponent):
     a64, b64 = a.astype(np.float64), b.astype(np.float64)
     bound = (k + 2) * U * (np.abs(a64) @ np.abs(b64)) + 6 * k * 2.0 ** -149
     assert np.all(np.abs(got - a64 @ b64) <= bound), float(np.max(np.abs(got - a64 @ b64) / bound))
+
+
+# Every kernel of three pieces: its shape, and whether A is stored along M.
+KERNELS = {"gemm_f32_b3_256x256": (4096, 4096, 64, False), "gemm_f32_b3_256x128": (4096, 2048, 64, False),
+           "gemm_f32_b3<": (2045, 1930, 77, False), "gemm_f32_b3kw": (1000, 1020, 1537, True),
+           "gemm_f32_b3sk": (2304, 2304, 256, False)}
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+@pytest.mark.parametrize("where,bits", [("a", 1), ("a", 0x7fff), ("a", 0x8000), ("a", 0x8001), ("b", 1),
+                                        ("b", 0x8000), ("alpha", 0x8000)])
+def test_least_subnormals(ctx, pool, kernel, where, bits):
+    """Operands of zeros and elements of at most `bits` least subnormals (2^-149), which bf16 rounds to
+    zero up to 0x8000 of them, stored so or made by alpha: every product counts."""
+    m, n, k, ta = KERNELS[kernel]
+    g = rng(9500 + bits)
+    small = lambda *s: np.ldexp(g.integers(-bits, bits + 1, s).astype(np.float64), -149).astype(np.float32)
+    large = lambda *s: np.ldexp(g.standard_normal(s), 100).astype(np.float32)
+    a, b = (large(m, k), small(k, n)) if where == "b" else (small(m, k), large(k, n))
+    alpha = 1.0
+    if where == "alpha":
+        a, alpha = np.ldexp(a, 40), 2.0 ** -40
+    got, name = _product(ctx, pool, a, b, ta, False, alpha)
+    assert name.startswith(kernel), name
+    _check(got, a, b, alpha, 0.0, None)
