@@ -9,10 +9,10 @@
 //
 // Elements are scaled by 2^23 before they are split and the sums by 2^-46 after: an f32, subnormals
 // included, is a whole multiple of 2^-149, so a scaled one is a whole multiple of 2^-126 and each of its pieces
-// zero or a normal bf16. So the pieces hold every element below 2^104 whole, whatever its size. A
-// workgroup whose scaled sums come out as anything but finite numbers (an infinity or a NaN in an operand,
-// an element of 2^104 or more, a sum of 2^82 or more: x - x0 turns an infinity into NaN) computes
-// its tile again with the f32 matrix instruction on the operands themselves (b3_redo).
+// zero or a normal bf16. So the pieces hold every element below 2^104 whole, whatever its size. Where
+// scaled sums come out as anything but finite numbers (an infinity or a NaN in an operand, an element of
+// 2^104 or more, a sum of 2^82 or more: x - x0 turns an infinity into NaN), the wave that holds them computes
+// their row of 32x32 blocks again with the f32 matrix instruction on the operands themselves (b3_redo).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -173,13 +173,6 @@ struct B3Loader {
     }
 };
 
-// The tile's sums in plain f32 (v_mfma_f32_32x32x2_f32), straight from memory: for tiles whose elements
-// the bf16 pieces do not cover. Slow and rare.
-template <int FM, int FN, int WN>
-__device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const float* B, uint32_t m0,
-                                                  uint32_t n0, uint32_t klen, int wave, int lane,
-                                                  floatx16 (&acc)[FM][FN]);
-
 // Every LDS access of this wave done, then the workgroup's barrier. Waves that load nothing store
 // nothing either, and only the fences tell the compiler that what they read there changes.
 __device__ __forceinline__ void b3_barrier() {
@@ -213,8 +206,8 @@ __device__ __forceinline__ void b3_block(const bf16x8 (&a)[3], const bf16x8 (&b)
 }
 
 // One (32 FM WM) x (32 FN WN) tile over k [0, klen) from A and B (batch plane, first k): acc, of the scaled
-// elements, negated where `sign` is -1.
-template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
+// elements, negated where `sign` is -1. ALONE: one wave per SIMD.
+template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE, bool ALONE = false>
 __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const float* A, const float* B,
                                         uint32_t m0, uint32_t n0, uint32_t klen, float sign, floatx16 (&acc)[FM][FN]) {
     constexpr int RA = 32 * FM * WM, RB = 32 * FN * WN;
@@ -267,9 +260,11 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
         auto step = [&](auto phase, uint32_t s) __attribute__((always_inline)) {
             constexpr int U = decltype(phase)::value, P = U & 1, X1 = (U + 1) % NX, X2 = (U + 2) % NX;
             constexpr int MG = 6 * FN;
-            // VALU instructions after each MFMA: a row takes 26, and the loop's own a few more.
+            // VALU instructions after each MFMA: a row takes 26, and the loop's own a few more. One more behind
+            // the barrier where nothing else covers a wave's wait there (4608 x 4608 x 512 on stream-K
+            // 150 -> 146 us, 2304^3 151 -> 148; 256x128 tiles of two waves per SIMD 167 against 173).
             constexpr int V = LOADS ? ((4 - EARLY) * 28 + (FM - 1) * MG - 1) / ((FM - 1) * MG) : 0;
-            constexpr int VL = LOADS ? (EARLY * 28 + MG - 1) / MG : 0;
+            constexpr int VL = LOADS ? (EARLY * 28 + MG - 1) / MG + (ALONE ? 1 : 0) : 0;
 #pragma unroll
             for (int i = 0; i + 1 < FM; ++i) {
                 read_a(a[(i + 1) & 1], i + 1, P);
@@ -365,42 +360,103 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
     }
 }
 
-template <int FM, int FN, int WN>
-__device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const float* B, uint32_t m0,
-                                                  uint32_t n0, uint32_t klen, int wave, int lane,
-                                                  floatx16 (&acc)[FM][FN]) {
-    const int wm = wave / WN, wn = wave % WN;
+// One wave's 32 x 32 FN outputs in plain f32 (v_mfma_f32_32x32x2_f32), straight from memory, for rows of
+// blocks whose scaled sums are not finite: rows from m, columns from n. Half h of the wave takes k 8 g + 4 h ..
+// 8 g + 4 h + 3 of group g, one 128-bit load an operand row where K is contiguous, four groups in
+// flight (the MFMAs of one take 256 FN cycles). Bound: the f32 matrix rate over the rows of blocks concerned, which it
+// reaches to about 60 %: 4096^3 with an infinity in one row of A 784 us, in every 64th 1270, with all of A NaN 1740
+// (601 without; 32-bit loads with nothing in flight took 3720, the f32 instruction alone 930); 3001 x 2011 x 1537
+// 238, 284 and 424 (132; 454), 2304^3 on stream-K 267, 317 and 481 (150; 190).
+template <int AM, int BMD, int FN>
+__device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const float* B, uint32_t m, uint32_t n,
+                                        uint32_t klen, int lane, floatx16 (&acc)[FN]) {
+    constexpr int D = 4;
     const uint32_t lr = lane & 31, h = lane >> 5;
     const float alpha_a = p.scale_b ? 1.0f : p.alpha, alpha_b = p.scale_b ? p.alpha : 1.0f;
-    const float *ar[FM], *br[FN];
+    // Uniform first elements and 32-bit byte offsets of the lane's (rows past the end repeat the last one).
+    A += static_cast<int64_t>(m) * p.a_sm;
+    B += static_cast<int64_t>(n) * p.b_sn;
+    const uint32_t ao = static_cast<uint32_t>((min(m + lr, p.m - 1) - m) * p.a_sm + 4 * h * p.a_sk) * 4u;
+    uint32_t bo[FN];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) ar[i] = A + static_cast<int64_t>(min(m0 + (wm * FM + i) * 32 + lr, p.m - 1)) * p.a_sm;
+    for (int j = 0; j < FN; ++j) {
+        bo[j] = static_cast<uint32_t>((min(n + j * 32 + lr, p.n - 1) - n) * p.b_sn + 4 * h * p.b_sk) * 4u;
+    }
+    const uint32_t groups = klen / 8;
+    floatx4 a[D], b[D][FN];
+    auto one = [](const float* q, uint32_t off) __attribute__((always_inline)) {
+        return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(q) + off);
+    };
+    auto get = [&](auto mode, const float* q, int64_t sk, uint32_t off) __attribute__((always_inline)) {
+        floatx4 x;
+        if constexpr (decltype(mode)::value == LOAD_K) {
+            x = *reinterpret_cast<const floatx4u*>(reinterpret_cast<const char*>(q) + off);
+        } else {
 #pragma unroll
-    for (int j = 0; j < FN; ++j) br[j] = B + static_cast<int64_t>(min(n0 + (wn * FN + j) * 32 + lr, p.n - 1)) * p.b_sn;
-    b3_zero(acc);
-    for (uint32_t k = 0; k < klen; k += 2) {
-        const uint32_t kk = k + h;
-        float a[FM], b[FN];
+            for (int e = 0; e < 4; ++e) x[e] = one(q + e * sk, off);
+        }
+        return x;
+    };
+    auto load = [&](uint32_t g, int u) __attribute__((always_inline)) {
+        const int64_t k = static_cast<int64_t>(min(g, groups - 1)) * 8;
+        a[u] = get(std::integral_constant<int, AM>{}, A + k * p.a_sk, p.a_sk, ao);
 #pragma unroll
-        for (int i = 0; i < FM; ++i) a[i] = kk < klen ? alpha_a * ar[i][kk * p.a_sk] : 0.0f;
+        for (int j = 0; j < FN; ++j) b[u][j] = get(std::integral_constant<int, BMD>{}, B + k * p.b_sk, p.b_sk, bo[j]);
+    };
+    auto multiply = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) b[j] = kk < klen ? alpha_b * br[j][kk * p.b_sk] : 0.0f;
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+            for (int j = 0; j < FN; ++j) {
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(alpha_a * a[u][e], alpha_b * b[u][j][e], acc[j], 0, 0, 0);
+            }
+    };
 #pragma unroll
-            for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+    if (groups > 0) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) load(u, u);
+        uint32_t g = 0;
+        for (; g + D <= groups; g += D) {
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                multiply(u);
+                load(g + D + u, u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < D; ++u)
+            if (g + u < groups) multiply(u);
+    }
+    if (groups * 8 < klen) {
+        const int64_t k = static_cast<int64_t>(groups) * 8;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool in = groups * 8 + 4 * h + e < klen;
+            a[0][e] = 0.0f;
+            if (in) a[0][e] = one(A + (k + e) * p.a_sk, ao);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                b[0][j][e] = 0.0f;
+                if (in) b[0][j][e] = one(B + (k + e) * p.b_sk, bo[j]);
+            }
+        }
+        multiply(0);
     }
 }
 
-// A tile's sums over k [0, klen), by whichever way holds its elements. The bf16 instruction cuts the
+// A tile's sums over k [0, klen). Returns the wave's rows of blocks (bit i: row i) whose sums are not finite and
+// that b3_redo has to compute. The bf16 instruction cuts the
 // bits that its accumulator has no room for, so a sum is a little low (2e-7 of it at K = 4096); `negative`
 // sums the negated products and negates the sum, which is then a little high: every other split of K does, and the
 // splits' errors cancel instead of adding up.
-template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE>
-__device__ __forceinline__ void b3_sums(const GemmArgs& p, char* smem, const float* A, const float* B, uint32_t m0,
+template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE, bool ALONE = false>
+__device__ __forceinline__ uint32_t b3_sums(const GemmArgs& p, char* smem, const float* A, const float* B, uint32_t m0,
                                         uint32_t n0, uint32_t klen, bool negative, int wave, int lane,
                                         floatx16 (&acc)[FM][FN]) {
-    b3_tile<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, negative ? -1.0f : 1.0f, acc);
+    b3_tile<AM, BMD, WM, WN, FM, FN, EDGE, ALONE>(p, smem, A, B, m0, n0, klen, negative ? -1.0f : 1.0f, acc);
     const float down = negative ? -B3_DOWN : B3_DOWN;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -411,9 +467,10 @@ __device__ __forceinline__ void b3_sums(const GemmArgs& p, char* smem, const flo
     // x * 0 is 0 unless x is infinite or NaN. Rows and columns past the output's edge hold
     // whatever the stages held, and do not count.
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
-    float z = 0.0f;
+    uint32_t bad = 0;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i) {
+        float z = 0.0f;
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
@@ -424,7 +481,9 @@ __device__ __forceinline__ void b3_sums(const GemmArgs& p, char* smem, const flo
                     z = z + t;
                 }
             }
-    if (__syncthreads_or(z != 0.0f)) b3_redo<FM, FN, WN>(p, A, B, m0, n0, klen, wave, lane, acc);
+        if (__any(z != 0.0f)) bad |= 1u << i;
+    }
+    return bad;
 }
 
 // gemm_f32_b3<AM, BMD, WM, WN, FM, FN, EDGE>: C = beta * C + sum_k (alpha * a) * b, or raw split-K partials,
@@ -454,17 +513,13 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
     const uint32_t klen = min(p.k - kb, p.k_chunk);
     const float* A = p.a + static_cast<int64_t>(bi) * p.a_sb + static_cast<int64_t>(kb) * p.a_sk;
     const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
-    floatx16 acc[FM][FN];
-    b3_zero(acc);
-    b3_sums<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, split & 1u, wave, lane, acc);
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
     float* C = p.partial != nullptr ? p.partial + static_cast<int64_t>(plane) * p.m * p.n
                                     : p.c + static_cast<int64_t>(bi) * p.c_sb;
     const int64_t c_sm = p.partial != nullptr ? static_cast<int64_t>(p.n) : p.c_sm;
     const int64_t c_sn = p.partial != nullptr ? 1 : p.c_sn;
     const float beta = p.partial != nullptr ? 0.0f : p.beta;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
+    auto store = [&](uint32_t i, const floatx16 (&x)[FN]) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
             const uint32_t col = n0 + (wn * FN + j) * 32 + lr;
@@ -473,11 +528,25 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
                 const uint32_t row = m0 + (wm * FM + i) * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
                 if (EDGE && (row >= p.m || col >= p.n)) continue;
                 float* q = C + row * c_sm + col * c_sn;
-                float v = acc[i][j][r];
+                float v = x[j][r];
                 if (beta != 0.0f) v = beta * *q + v;
                 *q = v;
             }
         }
+    };
+    floatx16 acc[FM][FN];
+    b3_zero(acc);
+    uint32_t bad = b3_sums<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, split & 1u, wave, lane, acc);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+        if ((bad >> i & 1u) == 0) store(i, acc[i]);
+    while (bad != 0) {
+        const uint32_t i = __builtin_ctz(bad);
+        bad &= bad - 1;
+        floatx16 t[FN];
+        b3_redo<AM, BMD, FN>(p, A, B, m0 + (wm * FM + i) * 32, n0 + wn * FN * 32, klen, lane, t);
+        store(i, t);
+    }
 }
 
 // gemm_f32_b3kw<AM, BMD, EDGE>: a 64x64 tile per workgroup, each of four waves summing the whole tile
@@ -603,17 +672,17 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     const int bm = wave >> 1, bn = wave & 1;
     const uint32_t col = n0 + bn * 32 + lr;
     auto row_of = [&](int r) { return m0 + bm * 32 + (r >> 2) * 8 + h * 4 + (r & 3); };
-    floatx16 v[1][1];
+    floatx16 v[1];
     float z = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const float* q = reinterpret_cast<const float*>(smem) + (wave * 16 + r) * 64 + lane;
-        v[0][0][r] = (q[0] + q[R * R]) + (q[2 * R * R] + q[3 * R * R]);
-        const float t = v[0][0][r] * 0.0f;
+        v[0][r] = (q[0] + q[R * R]) + (q[2 * R * R] + q[3 * R * R]);
+        const float t = v[0][r] * 0.0f;
         if (!EDGE || (row_of(r) < p.m && col < p.n)) z = z + t;
     }
     // (Each wave's own block, over the whole chunk.)
-    if (__syncthreads_or(z != 0.0f)) b3_redo<1, 1, 2>(p, A, B, m0, n0, klen, wave, lane, v);
+    if (__any(z != 0.0f)) b3_redo<AM, BMD, 1>(p, A, B, m0 + bm * 32, n0 + bn * 32, klen, lane, v);
     float* C = p.partial != nullptr ? p.partial + static_cast<int64_t>(plane) * p.m * p.n
                                     : p.c + static_cast<int64_t>(bi) * p.c_sb;
     const int64_t c_sm = p.partial != nullptr ? static_cast<int64_t>(p.n) : p.c_sm;
@@ -623,7 +692,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     for (int r = 0; r < 16; ++r) {
         if (EDGE && (row_of(r) >= p.m || col >= p.n)) continue;
         float* q = C + row_of(r) * c_sm + col * c_sn;
-        float x = v[0][0][r];
+        float x = v[0][r];
         if (beta != 0.0f) x = beta * *q + x;
         *q = x;
     }
@@ -671,7 +740,13 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_b3sk(GemmArgs p) {
         const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
         floatx16 acc[FM][FN];
         b3_zero(acc);
-        b3_sums<AM, BMD, 2, 2, FM, FN, false>(p, smem, A, B, m0, n0, len * STEP, false, wave, lane, acc);
+        const uint32_t bad = b3_sums<AM, BMD, 2, 2, FM, FN, false, true>(p, smem, A, B, m0, n0, len * STEP, false, wave, lane, acc);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            if ((bad >> i & 1u) != 0) {
+                b3_redo<AM, BMD, FN>(p, A, B, m0 + ((wave >> 1) * FM + i) * 32, n0 + (wave & 1) * FN * 32, len * STEP, lane, acc[i]);
+            }
+        }
         if (whole) {
             pl_store_c<FN>(p, acc, bi, m0, n0);
         } else {

@@ -3,6 +3,8 @@
 Every product is compared with the exact one in f64 under the bound of an f32 dot product,
 (K + 2) u sum |a||b| plus C's own rounding.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -164,3 +166,30 @@ def test_least_subnormals(ctx, pool, kernel, where, bits):
     got, name = _product(ctx, pool, a, b, ta, False, alpha)
     assert name.startswith(kernel), name
     _check(got, a, b, alpha, 0.0, None)
+
+
+@pytest.mark.parametrize("shape,kernel", [((4096, 4096, 4096), "gemm_f32_b3_256x256"), ((3001, 2011, 1537), "gemm_f32_b3<"),
+                                          ((2304, 2304, 2304), "gemm_f32_b3sk")])
+@pytest.mark.parametrize("value,every,limit", [(1e-35, 16, 2.0), (np.inf, 64, 3.5)])
+def test_time_with_elements_at_the_ends_of_the_range(ctx, pool, shape, kernel, value, every, limit):
+    """One tiny element in every sixteenth row of A costs nothing and an infinity in every 64th, half of all rows
+    of blocks, about one more pass: twice the time was measured, six to eleven times where whole tiles are computed again
+    with nothing in flight."""
+    m, n, k = shape
+    g = rng(9600)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+    B, Cc = Tensor(pool, Layout.dense([k, n]), b.ravel()), Tensor(pool, Layout.dense([m, n]), np.zeros(m * n, np.float32))
+    times = []
+    for special in (False, True):
+        if special:
+            a[::every, 7] = value
+        A = Tensor(pool, Layout.dense([m, k]), a.ravel())
+        best = np.inf
+        for _ in range(12):
+            t = time.perf_counter()
+            C.gemm(ctx, 1.0, A.view(), B.view(), 0.0, Cc.view())
+            best = min(best, time.perf_counter() - t)
+        times.append(best)
+        assert ctx.launches()[-1].startswith(kernel)
+    assert times[1] < limit * times[0], times
