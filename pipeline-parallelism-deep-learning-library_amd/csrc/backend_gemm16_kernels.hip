@@ -221,8 +221,11 @@ __global__ __launch_bounds__(QT) void gemm16_seq(Gemm16SeqArgs p) {
 // wherever the product itself needs no rounding, and that is the rule here: f16 elements have 11
 // significant bits and bf16 ones 8, so (alpha * a) * b has at most 24 when alpha has at most 2 or 8
 // (1, -0.5, 0.75, ...; the host's chain_fuses), and f16 products cannot leave f32's range. bf16
-// ones can, so a tile that meets an |alpha * a| or |b| outside [2^-55, 2^62) that is not zero is computed
-// again with separate multiplies and adds (`odd`).
+// ones can, so a slice that holds an |alpha * a| or |b| outside [2^-55, 2^62) that is not zero takes separate
+// multiplies and adds from the same stage (multiply_odd), at the VALU's rate: softmax weights and small gradients
+// are there as a matter of course. us, one such element / some in every slice / gemm16_seq: 2048 x 4096 x 1024
+// 162 / 365 / 420 (165 without any), 1501 x 1477 x 1023 75 / 171 / 174 (73), 128 x 1408 x 1024 17 / 51 / 128 (14.6); with
+// whole tiles computed again from memory 763 / 642, 354 / 360 and 185 / 186.
 // A last slice that is not full is padded with products (-0) * 1: adding -0 changes no sum.
 //
 // 32 NB x 32 NB outputs per 256-thread workgroup, four waves in 2 x 2 of NB x NB blocks of 16x16. All
@@ -250,6 +253,7 @@ __global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
     constexpr int R = 32 * NB, BK = 2048 / R, KG = BK / 16;
     constexpr int OP = R * BK;  // floats of one operand's stage
     __shared__ __attribute__((aligned(16))) float stage[2][2 * OP];
+    __shared__ uint32_t odd_slice[2];  // of each stage: 1 + the last slice with an element whose products may round
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, lr = lane & 15, lk = lane >> 4;
     // Tiles in groups of eight rows, each XCD (workgroups go round the eight in turn) a run of them.
@@ -257,26 +261,27 @@ __global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
     const uint32_t lin = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (blockIdx.x >> 3);
     const uint32_t group = lin / (8 * p.tiles_n), gm = min(p.tiles_m - group * 8, 8u), in = lin - group * 8 * p.tiles_n;
     const uint32_t m0 = (group * 8 + in % gm) * R, n0 = (in / gm) * R;
-    bool odd = false;  // an element whose products may round was met
 
     f32x4 acc[NB][NB];
-    // Output (i, j, r) of this lane, and the chain's start.
-    auto row_of = [&](int i, int r) { return m0 + (wm * NB + i) * 16 + lk * 4 + r; };
-    auto col_of = [&](int j) { return n0 + (wn * NB + j) * 16 + lr; };
-    auto start = [&]() __attribute__((always_inline)) {
+    // Output (i, j, r) of this lane.
+    const uint32_t row0 = m0 + wm * NB * 16 + lk * 4, col0 = n0 + wn * NB * 16 + lr;
+    auto row_of = [&](int i, int r) { return row0 + i * 16 + r; };
+    auto col_of = [&](int j) { return col0 + j * 16; };
 #pragma unroll
-        for (int i = 0; i < NB; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
-            for (int j = 0; j < NB; ++j)
+        for (int j = 0; j < NB; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    acc[i][j][r] = 0.0f;
-                    if (p.beta != 0.0f && row_of(i, r) < p.m && col_of(j) < p.n) {
-                        acc[i][j][r] = p.beta * widen<HK>(p.c[static_cast<int64_t>(row_of(i, r)) * p.c_sm + col_of(j)]);
-                    }
+            for (int r = 0; r < 4; ++r) {
+                acc[i][j][r] = 0.0f;
+                if (p.beta != 0.0f && row_of(i, r) < p.m && col_of(j) < p.n) {
+                    acc[i][j][r] = p.beta * widen<HK>(p.c[static_cast<int64_t>(row_of(i, r)) * p.c_sm + col_of(j)]);
                 }
-    };
-    start();
+            }
+    if constexpr (HK == 1) {
+        if (tid < 2) odd_slice[tid] = 0;
+        __syncthreads();
+    }
     const uint32_t slices = (p.k + BK - 1) / BK;
     auto loop = [&](auto vec, const uint16_t* src, int64_t s_row, int64_t s_k, uint32_t rows, float scale,
                     float pad, float* to) __attribute__((always_inline)) {
@@ -329,14 +334,16 @@ __global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
                 f[j] = scale * widen<HK>(h);
             }
             if constexpr (HK == 1) {
-                uint32_t low = 0xffffffffu, high = 0;
+                // Two instructions an element: twice the magnitude's bits less one (zero: the largest), and the
+                // least of three; the largest magnitude of three, in which NaNs do not count (nor need they).
+                uint32_t low = 0xffffffffu;
+                float high = 0.0f;
 #pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const uint32_t u = __builtin_bit_cast(uint32_t, f[j]) << 1;
-                    low = min(low, u - 1);  // zero: the largest
-                    high = max(high, u);
+                for (int j = 0; j < 16; j += 2) {
+                    low = min(low, min((__builtin_bit_cast(uint32_t, f[j]) << 1) - 1, (__builtin_bit_cast(uint32_t, f[j + 1]) << 1) - 1));
+                    __asm__("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(high) : "v"(f[j]), "v"(f[j + 1]));
                 }
-                odd = odd || low < ((127u - 55u) << 24) - 1 || high >= ((127u + 62u) << 24);
+                if (__any(low < ((127u - 55u) << 24) - 1 || high >= 0x1p62f)) odd_slice[s & 1] = s + 1;
             }
             if (k + 16 > p.k) {
 #pragma unroll
@@ -347,65 +354,117 @@ __global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(q + c * 4 * R) = f32x4{f[c], f[4 + c], f[8 + c], f[12 + c]};
         };
-        auto multiply = [&](uint32_t s) __attribute__((always_inline)) {
+        // A slice's fragments, read before the conversions of the next one and multiplied behind them.
+        f32x4 fa[KG][NB], fb[KG][NB];
+        auto read = [&](uint32_t s) __attribute__((always_inline)) {
             const float* as = stage[s & 1] + lk * 4 * R + (wm * NB * 16 + lr) * 4;
             const float* bs = stage[s & 1] + OP + lk * 4 * R + (wn * NB * 16 + lr) * 4;
 #pragma unroll
             for (int g = 0; g < KG; ++g) {
-                f32x4 a[NB], b[NB];
 #pragma unroll
-                for (int i = 0; i < NB; ++i) a[i] = *reinterpret_cast<const f32x4*>(as + g * 16 * R + i * 64);
+                for (int i = 0; i < NB; ++i) fa[g][i] = *reinterpret_cast<const f32x4*>(as + g * 16 * R + i * 64);
 #pragma unroll
-                for (int j = 0; j < NB; ++j) b[j] = *reinterpret_cast<const f32x4*>(bs + g * 16 * R + j * 64);
+                for (int j = 0; j < NB; ++j) fb[g][j] = *reinterpret_cast<const f32x4*>(bs + g * 16 * R + j * 64);
+            }
+        };
+        auto multiply = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < KG; ++g)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
                     for (int i = 0; i < NB; ++i)
 #pragma unroll
-                        for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+                        for (int j = 0; j < NB; ++j) {
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[g][i][e], fb[g][j][e], acc[i][j], 0, 0, 0);
+                        }
+        };
+        // The same slice as the chain is written: k by k, the next one's operands (past the last the first's
+        // again) read behind its sums.
+        auto multiply_odd = [&](uint32_t s) __attribute__((always_inline)) {
+            const float* as = stage[s & 1] + (wm * NB * 16 + lk * 4) * 4;
+            const float* bs = stage[s & 1] + OP + (wn * NB * 16 + lr) * 4;
+            float a[2][NB * 4], b[2][NB];
+            auto read = [&](int k, int to) __attribute__((always_inline)) {
+                const int at = (k >> 4) * 16 * R + (k & 3) * 4 * R + ((k >> 2) & 3);
+#pragma unroll
+                for (int i = 0; i < NB * 4; ++i) a[to][i] = as[at + ((i >> 2) * 16 + (i & 3)) * 4];
+#pragma unroll
+                for (int j = 0; j < NB; ++j) b[to][j] = bs[at + j * 64];
+            };
+            read(0, 0);
+#pragma unroll 1
+            for (int k = 0; k < BK; k += 4) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    read((k + u + 1) % BK, (u + 1) & 1);
+#pragma unroll
+                    for (int i = 0; i < NB * 4; ++i)
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) {
+                            const float prod = a[u & 1][i] * b[u & 1][j];
+                            acc[i >> 2][j][i & 3] = acc[i >> 2][j][i & 3] + prod;
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         };
         load(0);
         put(0);
         if (slices > 1) load(1);
         __syncthreads();
-        for (uint32_t s = 0; s < slices; ++s) {
+        auto next = [&](uint32_t s) __attribute__((always_inline)) {
             if (s + 1 < slices) put(s + 1);
             if (s + 2 < slices) load(s + 2);
-            multiply(s);
-            __syncthreads();
+        };
+        uint32_t s = 0;
+        if constexpr (HK == 0) {
+            for (; s < slices; ++s) {
+                read(s);
+                next(s);
+                multiply();
+                __syncthreads();
+            }
+        } else while (s < slices) {
+            bool odd = false;
+            for (; s < slices && !odd; ++s) {
+                const uint32_t last = odd_slice[s & 1];
+                read(s);
+                next(s);
+                odd = __builtin_amdgcn_readfirstlane(last) == s + 1;
+                if (odd) {
+                    multiply_odd(s);
+                    // The MFMAs that follow add (-0) * 1, which changes no sum. (A branch around them takes 4 % of all
+                    // other slices' time.)
+#pragma unroll
+                    for (int g = 0; g < KG; ++g)
+#pragma unroll
+                        for (int i = 0; i < NB; ++i) {
+                            fa[g][i] = f32x4{-0.0f, -0.0f, -0.0f, -0.0f};
+                            fb[g][i] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+                        }
+                }
+                multiply();
+                __syncthreads();
+            }
+            // Where one slice holds such elements the next ones mostly do too.
+            for (; s < slices && __builtin_amdgcn_readfirstlane(odd_slice[s & 1]) == s + 1; ++s) {
+                next(s);
+                multiply_odd(s);
+                __syncthreads();
+            }
         }
     };
-    if (wave < 2) {
+    if (wave < 2 && p.alpha == 1.0f) {
+        // (One multiplication an element less: 4096^3 1220 -> 1200 us.)
+        loop(std::integral_constant<bool, AV>{}, p.a + static_cast<int64_t>(m0) * p.a_sm, p.a_sm, p.a_sk, p.m - m0,
+             1.0f, -0.0f, stage[0]);
+    } else if (wave < 2) {
         loop(std::integral_constant<bool, AV>{}, p.a + static_cast<int64_t>(m0) * p.a_sm, p.a_sm, p.a_sk, p.m - m0,
              p.alpha, -0.0f, stage[0]);
     } else {
         loop(std::integral_constant<bool, BV>{}, p.b + static_cast<int64_t>(n0) * p.b_sn, p.b_sn, p.b_sk, p.n - n0,
              1.0f, 1.0f, stage[0] + OP);
-    }
-
-    if (HK == 1 && __syncthreads_or(odd)) {
-        // Slow and rare: the chain as written, every element from memory.
-        start();
-        const uint16_t *ar[NB * 4], *br[NB];
-#pragma unroll
-        for (int i = 0; i < NB * 4; ++i) ar[i] = p.a + static_cast<int64_t>(min(row_of(i >> 2, i & 3), p.m - 1)) * p.a_sm;
-#pragma unroll
-        for (int j = 0; j < NB; ++j) br[j] = p.b + static_cast<int64_t>(min(col_of(j), p.n - 1)) * p.b_sn;
-        for (uint32_t k = 0; k < p.k; ++k) {
-            float bv[NB];
-#pragma unroll
-            for (int j = 0; j < NB; ++j) bv[j] = widen<HK>(br[j][k * p.b_sk]);
-#pragma unroll
-            for (int i = 0; i < NB * 4; ++i) {
-                const float av = p.alpha * widen<HK>(ar[i][k * p.a_sk]);
-#pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    const float prod = av * bv[j];
-                    acc[i >> 2][j][i & 3] = acc[i >> 2][j][i & 3] + prod;
-                }
-            }
-        }
     }
 
 #pragma unroll

@@ -1,11 +1,13 @@
 """The 16-bit Backend gemm on the f32 matrix cores (gemm16_chain): CpuBackend's bits at the
 edges of its tiles and slices and of the range in which its products need no rounding."""
+import time
+
 import numpy as np
 import pytest
 
 import oracle
 from helpers import rng
-from test_backend_gpu import run16, same16, hb  # noqa: F401  (hb: the backend fixture)
+from test_backend_gpu import run16, same16, hb, up16  # noqa: F401  (hb: the backend fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +59,47 @@ def test_bf16_exponents_whose_products_round(hb, alpha, low, high):
     b[bt] = np.ldexp(b[bt], g.integers(low, high + 1, 40))
     with np.errstate(over="ignore"):
         _check(hb, "bf16", "bt", a, b, g.standard_normal((m, n)), m, k, n, alpha, 0.5)
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 330, 100), (1500, 167, 1450), (2900, 83, 2820)])
+@pytest.mark.parametrize("layout", ["bt", "at"])
+def test_bf16_slices_whose_products_round(hb, m, k, n, layout):
+    """32x32, 64x64 and 128x128 tiles with such slices alone, in runs, first and last, among slices
+    whose products need no rounding: either way of a slice continues the other's sums."""
+    g = rng(8950 + m)
+    a, b = g.standard_normal((m, k)), g.standard_normal((k, n))
+    for k0, k1 in ((0, 1), (k // 3, k // 3 + 1), (k // 2, 3 * k // 4), (k - 1, k)):
+        rows = g.integers(0, m, m // 8 + 1)
+        a[rows, k0:k1] = np.ldexp(a[rows, k0:k1], -140)
+        b[k0:k1, g.integers(0, n, 9)] *= 2.0 ** -60
+    a[3] = np.ldexp(a[3], -100)  # sums of products below the normal range alone
+    b[:, 5] = np.ldexp(b[:, 5], -40)
+    _check(hb, "bf16", layout, a, b, g.standard_normal((m, n)), m, k, n, 0.75, 0.0)
+
+
+@pytest.mark.parametrize("m,k,n", [(2048, 1024, 4096), (1501, 1023, 1477)])
+def test_time_with_bf16_elements_whose_products_round(hb, m, k, n):
+    """One element of 1e-20 costs next to nothing (1.0 of the time without was measured), one in every slice
+    of every tile the VALU's rate (2.2 to 2.4; whole tiles computed again took 4.5 times in both)."""
+    g = rng(8960)
+    a = np.ascontiguousarray(g.standard_normal((m, k), dtype=np.float32))
+    b = up16(hb, "bf16", oracle.f32_to_bf16(g.standard_normal(k * n, dtype=np.float32)), (k, n))
+    c = up16(hb, "bf16", np.zeros(m * n, np.uint16), (m, n))
+    times = []
+    for what in ("none", "one", "all"):
+        if what == "one":
+            a[m // 2, k // 2] = 1e-20
+        elif what == "all":
+            a[::16] = 1e-20
+        t16 = up16(hb, "bf16", oracle.f32_to_bf16(a.ravel()), (m, k))
+        hb.gemm(t16, b, c, 1.0, 0.0)
+        hb.sync()
+        best = np.inf
+        for _ in range(12):
+            t = time.perf_counter()
+            for _ in range(4):
+                hb.gemm(t16, b, c, 1.0, 0.0)
+            hb.sync()
+            best = min(best, time.perf_counter() - t)
+        times.append(best)
+    assert times[1] < 1.6 * times[0] and times[2] < 3.2 * times[0], times
