@@ -51,6 +51,12 @@ struct B3Geo {
 // instead, with the tile computed again where one is too small, cost as much per element and 4096^3 with
 // one element of 1e-35 4028 us, against 600 with the scale.
 constexpr float B3_UP = 0x1p23f, B3_DOWN = 0x1p-46f;
+// Slices after which a tile's sums change sign (see b3_sums): within the loop, a multiple of its unrolling, or by
+// another loop around it for one wave per SIMD, whose schedule the first way disturbs (2304^3 on stream-K 148 ->
+// 153 us) and whose registers take the second (all other tiles would spill: 2048^3 97 -> 112 us). That loop costs 3 %
+// at K = 1024 (3072 x 3072 120 -> 124 us), so it has a kernel of its own for K beyond one turn.
+constexpr uint32_t B3_TURN = 64, B3_TURN_ALONE = 256;
+enum B3Turns { TURNS_INSIDE, TURNS_NONE, TURNS_AROUND };
 
 // (x, y) -> three packed pairs of bf16 pieces. Eleven VALU instructions a pair and two for the scale, four
 // cycles each, and up to six of them hide behind every MFMA. (v_dot2_f32_bf16 would do the subtraction and the
@@ -205,10 +211,20 @@ __device__ __forceinline__ void b3_block(const bf16x8 (&a)[3], const bf16x8 (&b)
     }
 }
 
+template <int FM, int FN>
+__device__ __forceinline__ void b3_scale(floatx16 (&acc)[FM][FN], float by) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = by * acc[i][j][r];
+}
+
 // One (32 FM WM) x (32 FN WN) tile over k [0, klen) from A and B (batch plane, first k): acc, of the scaled
-// elements, negated where `sign` is -1. ALONE: one wave per SIMD.
-template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE, bool ALONE = false>
-__device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const float* A, const float* B,
+// elements, added to acc, and of the sign returned. `sign` is the first slices'. ALONE: one wave per SIMD, one sign.
+template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE, bool ALONE>
+__device__ __forceinline__ float b3_tile(const GemmArgs& p, char* smem, const float* A, const float* B,
                                         uint32_t m0, uint32_t n0, uint32_t klen, float sign, floatx16 (&acc)[FM][FN]) {
     constexpr int RA = 32 * FM * WM, RB = 32 * FN * WN;
     using GA = B3Geo<RA>;
@@ -226,7 +242,7 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
     const uint32_t fb = fr * GB::CLS + fq + fh * GB::CH + wn * FN * 128 + GA::BYTES;
     const uint32_t full = klen / B3_BK, left = klen - full * B3_BK;
 
-    auto loop = [&](auto* loader, float scale, char* mine) __attribute__((always_inline)) {
+    auto loop = [&](auto* loader, float scale, float turned, char* mine) __attribute__((always_inline)) {
         using LD = std::remove_pointer_t<decltype(loader)>;
         constexpr bool LOADS = !std::is_same_v<LD, void*>;
         // Slice s passes through the registers x[s % NX] into stage s % 2. Step s multiplies slice s. All
@@ -245,8 +261,13 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
                 else loader->load(to);
             }
         };
-        auto put_row = [&](int i, int stage, const B3Block& from) __attribute__((always_inline)) {
-            if constexpr (LOADS) loader->store_row(mine + stage * ST, from, i, scale);
+        // Row i of slice s's block, scaled by `scale` or, every other B3_TURN slices, `turned`.
+        constexpr uint32_t TURN = ALONE ? 0 : B3_TURN;
+        auto put_row = [&](int i, uint32_t s, int stage, const B3Block& from) __attribute__((always_inline)) {
+            if constexpr (LOADS) loader->store_row(mine + stage * ST, from, i, (s & TURN) != 0 ? turned : scale);
+        };
+        auto turn = [&](uint32_t s) __attribute__((always_inline)) {
+            if (TURN != 0 && s % B3_TURN == 0 && s != 0 && s < slices) b3_scale(acc, -1.0f);
         };
         bf16x8 a[2][3], b[FN][3];
         auto read_a = [&](bf16x8 (&to)[3], int i, int stage) __attribute__((always_inline)) {
@@ -271,7 +292,7 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
                 // This row of blocks' share of the conversion.
 #pragma unroll
                 for (int r = EARLY + i * (4 - EARLY) / (FM - 1); r < EARLY + (i + 1) * (4 - EARLY) / (FM - 1); ++r) {
-                    put_row(r, P ^ 1, x[X1]);
+                    put_row(r, s + 1, P ^ 1, x[X1]);
                 }
                 b3_block<FN>(a[i & 1], b, acc[i], [](int) {});
                 // One read after each of the first MFMAs, the conversion's VALU work and writes spread over all.
@@ -289,7 +310,7 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
             b3_barrier();
             constexpr int L = (FM - 1) & 1;
 #pragma unroll
-            for (int r = 0; r < EARLY; ++r) put_row(r, P, x[X2]);
+            for (int r = 0; r < EARLY; ++r) put_row(r, s + 2, P, x[X2]);
             b3_block<FN>(a[L], b, acc[FM - 1], [&](int t) {
                 if (t == 0) read_b(2, P ^ 1);
                 if (t == 2) {
@@ -318,9 +339,9 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
 #pragma unroll
         for (int s = 0; s < NX; ++s) fetch(s, x[s]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) put_row(r, 0, x[0]);
+        for (int r = 0; r < 4; ++r) put_row(r, 0, 0, x[0]);
 #pragma unroll
-        for (int r = 0; r < EARLY; ++r) put_row(r, 1, x[1]);
+        for (int r = 0; r < EARLY; ++r) put_row(r, 1, 1, x[1]);
         fetch(NX, x[0]);
         b3_barrier();
         read_a(a[0], 0, 0);
@@ -330,34 +351,41 @@ __device__ __forceinline__ void b3_tile(const GemmArgs& p, char* smem, const flo
         uint32_t s = 0;
         if constexpr (NX == 4) {
             for (; s + 3 < slices; s += 4) {
+                turn(s);
                 step(std::integral_constant<int, 0>{}, s);
                 step(std::integral_constant<int, 1>{}, s + 1);
                 step(std::integral_constant<int, 2>{}, s + 2);
                 step(std::integral_constant<int, 3>{}, s + 3);
             }
+            turn(s);
             if (s < slices) step(std::integral_constant<int, 0>{}, s);
             if (s + 1 < slices) step(std::integral_constant<int, 1>{}, s + 1);
             if (s + 2 < slices) step(std::integral_constant<int, 2>{}, s + 2);
         } else {
             for (; s + 1 < slices; s += 2) {
+                turn(s);
                 step(std::integral_constant<int, 0>{}, s);
                 step(std::integral_constant<int, 1>{}, s + 1);
             }
+            turn(s);
             if (s < slices) step(std::integral_constant<int, 0>{}, s);
         }
     };
     if (wave < WA) {
         B3Loader<AM, RA, EDGE> ld;
         ld.init(A, p.a_sm, p.a_sk, m0, p.m, tid);
-        loop(&ld, sign * (p.scale_b ? B3_UP : B3_UP * p.alpha), smem);
+        const float scale = sign * (p.scale_b ? B3_UP : B3_UP * p.alpha);
+        loop(&ld, scale, -scale, smem);
     } else if (wave < WA + WB) {
         B3Loader<BMD, RB, EDGE> ld;
         ld.init(B, p.b_sn, p.b_sk, n0, p.n, tid - RA);
-        loop(&ld, p.scale_b ? B3_UP * p.alpha : B3_UP, smem + GA::BYTES);
+        const float scale = p.scale_b ? B3_UP * p.alpha : B3_UP;
+        loop(&ld, scale, scale, smem + GA::BYTES);
     } else {
         void* none = nullptr;
-        loop(&none, 1.0f, smem);
+        loop(&none, 1.0f, 1.0f, smem);
     }
+    return !ALONE && (full + (left != 0) - 1 & B3_TURN) != 0 ? -sign : sign;
 }
 
 // One wave's 32 x 32 FN outputs in plain f32 (v_mfma_f32_32x32x2_f32), straight from memory, for rows of
@@ -448,22 +476,32 @@ __device__ __forceinline__ void b3_redo(const GemmArgs& p, const float* A, const
 }
 
 // A tile's sums over k [0, klen). Returns the wave's rows of blocks (bit i: row i) whose sums are not finite and
-// that b3_redo has to compute. The bf16 instruction cuts the
-// bits that its accumulator has no room for, so a sum is a little low (2e-7 of it at K = 4096); `negative`
-// sums the negated products and negates the sum, which is then a little high: every other split of K does, and the
-// splits' errors cancel instead of adding up.
-template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE, bool ALONE = false>
+// that b3_redo has to compute. The bf16 instruction rounds down where its accumulator has no room, so a sum over
+// one sign is a little low: 2.7e-7 of it at K = 4096 on normal operands, 1e-5 at 262144. `negative` sums the negated
+// products and negates the sum, which is then a little high: every other split of K does, and so
+// does every other B3_TURN slices of a longer K, and the errors cancel instead of adding up. Error against f64,
+// normal operands, 2048^2 outputs, over one sign / now / f32 instruction: K = 4096 1.00e-6 / 0.97e-6 / 1.15e-6, 16384
+// 2.1e-6 / 1.9e-6 / 2.3e-6, 65536 4.5e-6 / 3.5e-6 / 4.6e-6, 262144 1.1e-5 / 6.3e-6 / 9.2e-6.
+template <int AM, int BMD, int WM, int WN, int FM, int FN, bool EDGE, B3Turns TURNS>
 __device__ __forceinline__ uint32_t b3_sums(const GemmArgs& p, char* smem, const float* A, const float* B, uint32_t m0,
                                         uint32_t n0, uint32_t klen, bool negative, int wave, int lane,
                                         floatx16 (&acc)[FM][FN]) {
-    b3_tile<AM, BMD, WM, WN, FM, FN, EDGE, ALONE>(p, smem, A, B, m0, n0, klen, negative ? -1.0f : 1.0f, acc);
-    const float down = negative ? -B3_DOWN : B3_DOWN;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = down * acc[i][j][r];
+    float sign = negative ? -1.0f : 1.0f;
+    if constexpr (TURNS == TURNS_AROUND) {
+        for (uint32_t k = 0;;) {
+            const uint32_t len = min(klen - k, B3_TURN_ALONE * B3_BK);
+            b3_tile<AM, BMD, WM, WN, FM, FN, EDGE, true>(p, smem, A + static_cast<int64_t>(k) * p.a_sk,
+                                                         B + static_cast<int64_t>(k) * p.b_sk, m0, n0, len, sign, acc);
+            k += len;
+            if (k == klen) break;
+            b3_scale(acc, -1.0f);
+            sign = -sign;
+            b3_barrier();  // every wave is done with the stages
+        }
+    } else {
+        sign = b3_tile<AM, BMD, WM, WN, FM, FN, EDGE, TURNS == TURNS_NONE>(p, smem, A, B, m0, n0, klen, sign, acc);
+    }
+    b3_scale(acc, sign * B3_DOWN);
     // x * 0 is 0 unless x is infinite or NaN. Rows and columns past the output's edge hold
     // whatever the stages held, and do not count.
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5;
@@ -536,7 +574,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
     };
     floatx16 acc[FM][FN];
     b3_zero(acc);
-    uint32_t bad = b3_sums<AM, BMD, WM, WN, FM, FN, EDGE>(p, smem, A, B, m0, n0, klen, split & 1u, wave, lane, acc);
+    uint32_t bad = b3_sums<AM, BMD, WM, WN, FM, FN, EDGE, TURNS_INSIDE>(p, smem, A, B, m0, n0, klen, split & 1u, wave, lane, acc);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
         if ((bad >> i & 1u) == 0) store(i, acc[i]);
@@ -698,11 +736,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     }
 }
 
-// gemm_f32_b3sk<AM, BMD>: gemm_f32_sk's runs, slots and tickets (gemm_pipe.h) over the three-piece
+// gemm_f32_b3sk<AM, BMD, TURNS>: gemm_f32_sk's runs, slots and tickets (gemm_pipe.h) over the three-piece
 // sums of full 128x128 tiles: each run's part of a tile is checked, and summed again where it must be, before
 // it meets the other run's. One workgroup per compute unit. 48^6 in rank 4 (2304^3): 185 -> 149 us, 164 TFLOP/s,
 // with one wave per SIMD; 2048^3, the same wave on whole tiles, 126 -> 98 us.
-template <int AM, int BMD>
+template <int AM, int BMD, B3Turns TURNS>
 __global__ __launch_bounds__(256, 1) void gemm_f32_b3sk(GemmArgs p) {
     constexpr int FM = 2, FN = 2, RA = 128, RB = 128, SLOT = 128 * 128, STEP = 128;
     constexpr int ST = B3Geo<RA>::BYTES + B3Geo<RB>::BYTES;
@@ -740,7 +778,7 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_b3sk(GemmArgs p) {
         const float* B = p.b + static_cast<int64_t>(bi) * p.b_sb + static_cast<int64_t>(kb) * p.b_sk;
         floatx16 acc[FM][FN];
         b3_zero(acc);
-        const uint32_t bad = b3_sums<AM, BMD, 2, 2, FM, FN, false, true>(p, smem, A, B, m0, n0, len * STEP, false, wave, lane, acc);
+        const uint32_t bad = b3_sums<AM, BMD, 2, 2, FM, FN, false, TURNS>(p, smem, A, B, m0, n0, len * STEP, false, wave, lane, acc);
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             if ((bad >> i & 1u) != 0) {

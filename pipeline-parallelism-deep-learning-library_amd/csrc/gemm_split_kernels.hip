@@ -40,7 +40,11 @@ void launch_sk(hipStream_t s, const GemmArgs& a, uint32_t groups) {
         fail_invalid("the stream-K GEMM needs full 128x128 tiles, at least one per range, K in whole steps "
                      "and its scratch");
     }
-    hipLaunchKernelGGL((gemm_f32_b3sk<AM, BMD>), dim3(groups), dim3(256), 0, s, a);
+    if (a.k > B3_TURN_ALONE * B3_BK) {
+        hipLaunchKernelGGL((gemm_f32_b3sk<AM, BMD, TURNS_AROUND>), dim3(groups), dim3(256), 0, s, a);
+    } else {
+        hipLaunchKernelGGL((gemm_f32_b3sk<AM, BMD, TURNS_NONE>), dim3(groups), dim3(256), 0, s, a);
+    }
 }
 
 }  // namespace
