@@ -466,7 +466,7 @@ def bench_backend_gemm16(events, args, timed_fn, m=4096, n=4096, k=4096):
     terms = m * n * k / (ms * 1e-3) / 1e12
     res = {"name": f"Backend::gemm f16 {m}x{n}x{k} (CpuBackend's f32 chain, bit-exact)", "ms": ms,
            "tterms": terms, "tflops_vector": 2 * terms, "frac_vector": 2 * terms / PEAK_VECTOR_TFLOPS,
-           "kernel": "gemm16_chain<0, 4, true, false>"}
+           "kernel": hb.debug_launches()[-1]}
     hb.close()
     if not args.no_cpu:
         rows = 4

@@ -507,8 +507,9 @@ bool chain_near(const Gemm16SeqArgs& a) {
     return near(a.a_sm, a.a_sk) && near(a.b_sn, a.b_sk);
 }
 
+// Launches the chain kernel; returns its name for the launch log.
 template <int HK>
-void launch_chain(hipStream_t s, Gemm16SeqArgs a) {
+const char* launch_chain(hipStream_t s, Gemm16SeqArgs a) {
     // The largest tiles whose grid still gives every compute unit two workgroups; the
     // smallest ones for anything less.
     uint32_t tile = 128;
@@ -519,9 +520,16 @@ void launch_chain(hipStream_t s, Gemm16SeqArgs a) {
     const uint64_t groups = gemm16_seq_workgroups(a.m, a.n, tile);
     if (groups == 0 || groups * 256 > 0xffffffffull) fail_invalid("16-bit gemm grid exceeds one launch");
     const uint32_t g = static_cast<uint32_t>(groups);
-    if (tile == 128) launch_chain_nb<HK, 4>(s, a, g);
-    else if (tile == 64) launch_chain_nb<HK, 2>(s, a, g);
-    else launch_chain_nb<HK, 1>(s, a, g);
+    if (tile == 128) {
+        launch_chain_nb<HK, 4>(s, a, g);
+        return HK == 1 ? "gemm_bf16_chain128" : "gemm_f16_chain128";
+    }
+    if (tile == 64) {
+        launch_chain_nb<HK, 2>(s, a, g);
+        return HK == 1 ? "gemm_bf16_chain64" : "gemm_f16_chain64";
+    }
+    launch_chain_nb<HK, 1>(s, a, g);
+    return HK == 1 ? "gemm_bf16_chain32" : "gemm_f16_chain32";
 }
 
 }  // namespace
@@ -537,9 +545,9 @@ void launch_gemm16_seq(Context* ctx, hipStream_t s, const Gemm16SeqArgs& args) {
         fail_invalid("16-bit gemm grid does not match its extents");
     }
     const dim3 grid(static_cast<uint32_t>(groups));
+    const char* name = args.kind == 1 ? "gemm_bf16_seq" : "gemm_f16_seq";
     if (args.k > 0 && chain_fuses(args.kind, args.alpha) && chain_near(args)) {
-        if (args.kind == 1) launch_chain<1>(s, args);
-        else launch_chain<0>(s, args);
+        name = args.kind == 1 ? launch_chain<1>(s, args) : launch_chain<0>(s, args);
     } else if (args.kind == 1) {
         if (args.tile == 64) {
             hipLaunchKernelGGL((gemm16_seq<1, 4>), grid, dim3(QT), 0, s, args);
@@ -553,8 +561,8 @@ void launch_gemm16_seq(Context* ctx, hipStream_t s, const Gemm16SeqArgs& args) {
             hipLaunchKernelGGL((gemm16_seq<0, 8>), grid, dim3(QT), 0, s, args);
         }
     }
-    check_hip(hipGetLastError(), "gemm16_seq");
-    note_launch(ctx, args.kind == 1 ? "gemm_bf16_seq" : "gemm_f16_seq");
+    check_hip(hipGetLastError(), name);
+    note_launch(ctx, name);
 }
 
 }  // namespace lg

@@ -17,9 +17,12 @@ def _bits(kind, x):
     return oracle.f32_to_f16(x) if kind == "f16" else oracle.f32_to_bf16(x)
 
 
-def _check(hb, kind, layout, a, b, c, m, k, n, alpha, beta):
+def _check(hb, kind, layout, a, b, c, m, k, n, alpha, beta, kernel):
+    """Bits against the oracle's, and the kernel that ran: a name, or the tile of the chain on the matrix cores."""
     a16, b16, c16 = _bits(kind, a.ravel()), _bits(kind, b.ravel()), _bits(kind, c.ravel())
     got = run16(hb, kind, layout, a16, b16, c16, m, k, n, alpha, beta)
+    name = hb.debug_launches()[-1]
+    assert name == (kernel if isinstance(kernel, str) else f"gemm_{kind}_chain{kernel}"), name
     want = oracle.gemm_seq_16(kind, alpha, beta, a16.reshape(m, k), b16.reshape(k, n), c16.reshape(m, n))
     assert same16(kind, got, want)
 
@@ -34,14 +37,14 @@ def test_tile_and_slice_edges(hb, kind, layout, m, k, n):
     g = rng(8800 + m + k + n)
     alpha, beta = [(1.0, 0.0), (-0.75, 0.3)][(m + k) % 2]
     _check(hb, kind, layout, g.standard_normal((m, k)), g.standard_normal((k, n)),
-           g.standard_normal((m, n)), m, k, n, alpha, beta)
+           g.standard_normal((m, n)), m, k, n, alpha, beta, 128 if m > 2000 else 64 if m > 1400 else 32)
 
 
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_negative_zero_sums_survive_the_padding(hb, kind):
     m, k, n = 40, 19, 36
     a, b, c = -np.zeros((m, k), np.float32), np.ones((k, n), np.float32), -np.zeros((m, n), np.float32)
-    _check(hb, kind, "plain", a, b, c, m, k, n, 1.0, 1.0)
+    _check(hb, kind, "plain", a, b, c, m, k, n, 1.0, 1.0, 32)
 
 
 @pytest.mark.parametrize("alpha", [1.0, 2.0 ** -10, 1.9921875, 0.3])
@@ -58,7 +61,8 @@ def test_bf16_exponents_whose_products_round(hb, alpha, low, high):
     bt = (g.integers(0, k, 40), g.integers(0, n, 40))
     b[bt] = np.ldexp(b[bt], g.integers(low, high + 1, 40))
     with np.errstate(over="ignore"):
-        _check(hb, "bf16", "bt", a, b, g.standard_normal((m, n)), m, k, n, alpha, 0.5)
+        _check(hb, "bf16", "bt", a, b, g.standard_normal((m, n)), m, k, n, alpha, 0.5,
+               "gemm_bf16_seq" if alpha == 0.3 else 32)
 
 
 @pytest.mark.parametrize("m,k,n", [(70, 330, 100), (1500, 167, 1450), (2900, 83, 2820)])
@@ -74,7 +78,7 @@ def test_bf16_slices_whose_products_round(hb, m, k, n, layout):
         b[k0:k1, g.integers(0, n, 9)] *= 2.0 ** -60
     a[3] = np.ldexp(a[3], -100)  # sums of products below the normal range alone
     b[:, 5] = np.ldexp(b[:, 5], -40)
-    _check(hb, "bf16", layout, a, b, g.standard_normal((m, n)), m, k, n, 0.75, 0.0)
+    _check(hb, "bf16", layout, a, b, g.standard_normal((m, n)), m, k, n, 0.75, 0.0, {70: 32, 1500: 64, 2900: 128}[m])
 
 
 @pytest.mark.parametrize("m,k,n", [(2048, 1024, 4096), (1501, 1023, 1477)])
