@@ -815,8 +815,9 @@ def test_wide_direct_load_batched_with_permuted_b(ctx, pool):
                                             (2040, 1932, 300, False, True, True),
                                             (2048, 1924, 260, True, True, False)])
 def test_two_wave_groups_per_workgroup(ctx, pool, m, n, k, ta, tb, tc):
-    """Grids of exactly 256 128x128 direct-load tiles (one workgroup per compute unit) run two
-    wave groups per workgroup, each on half of the K slices, their sums added in group order:
+    """Grids of exactly 256 128x128 direct-load tiles (one workgroup per compute unit), planned with two
+    wave groups per workgroup and run on the three-piece kernel's one (the groups run for wide pitches,
+    test_wide_pitch_gpu.py):
     ragged M and N edges, K not in whole steps of the pipelined kernel (K = 1936), odd slice
     counts (the second group one slice short: K = 1004, 63 slices; K = 260, 17), partial last
     slices (K = 1004, 300, 260), every operand layout, and C
@@ -837,6 +838,7 @@ def test_two_wave_groups_per_workgroup(ctx, pool, m, n, k, ta, tb, tc):
     Cc.upload()
     C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
     assert np.array_equal(first.view(np.uint32), Cc.read().view(np.uint32))
+    assert [x for x in ctx.launches() if x.startswith("gemm")][-1].startswith("gemm_f32_b3<")
     _gemm_fast_check(f"two groups {m}x{n}x{k} ta={ta} tb={tb} tc={tc}", first, A.host, la,
                      B.host, lb, c0, lc, m, n, k, alpha, beta)
 
@@ -847,7 +849,8 @@ def test_two_wave_groups_per_workgroup(ctx, pool, m, n, k, ta, tb, tc):
                                             (964, 1024, 516, True, True, False)])
 def test_four_wave_groups_on_64x64_tiles(ctx, pool, m, n, k, ta, tb, tc):
     """Grids of exactly 256 64x64 tiles (a 128x128 grid would need split-K) on the direct-load
-    kernel with four wave groups of 32-deep slices: ragged edges, K not in whole steps of the
+    kernel with four wave groups of 32-deep slices where A lies along K, on the three-piece kernel's four waves
+    where it lies along M: ragged edges, K not in whole steps of the
     K-split kernel (K = 1000), groups with fewer slices than the others (K = 900: 8, 8, 8, 5
     slices; K = 516: 5, 5, 5, 2), partial last slices,
     every operand layout and C column-major, against crates/cpu on every element; the same
@@ -868,6 +871,7 @@ def test_four_wave_groups_on_64x64_tiles(ctx, pool, m, n, k, ta, tb, tc):
     Cc.upload()
     C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
     assert np.array_equal(first.view(np.uint32), Cc.read().view(np.uint32))
+    assert [x for x in ctx.launches() if x.startswith("gemm")][-1].startswith("gemm_f32_b3kw<" if ta else "gemm_f32_dl<")
     _gemm_fast_check(f"four groups {m}x{n}x{k} ta={ta} tb={tb} tc={tc}", first, A.host, la,
                      B.host, lb, c0, lc, m, n, k, alpha, beta)
 
@@ -898,6 +902,7 @@ def test_k_split_waves_on_64x64_tiles(ctx, pool, m, n, k, ta, tb, tc):
     Cc.upload()
     C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
     assert np.array_equal(first.view(np.uint32), Cc.read().view(np.uint32))
+    assert [x for x in ctx.launches() if x.startswith("gemm")][-1].startswith("gemm_f32_kw<")
     _gemm_fast_check(f"k-split waves {m}x{n}x{k} ta={ta} tb={tb} tc={tc}", first, A.host, la,
                      B.host, lb, c0, lc, m, n, k, alpha, beta)
 
@@ -928,6 +933,7 @@ def test_k_split_waves_split_along_k(ctx, pool, m, n, k, ta, tb, tc, splits):
     Cc.upload()
     C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
     assert np.array_equal(first.view(np.uint32), Cc.read().view(np.uint32))
+    assert [x for x in ctx.launches() if x.startswith("gemm")][-1].startswith("gemm_f32_kw<")
     _gemm_fast_check(f"k-split waves, split {m}x{n}x{k} ta={ta} tb={tb} tc={tc}", first, A.host, la,
                      B.host, lb, c0, lc, m, n, k, alpha, beta)
 
@@ -935,7 +941,7 @@ def test_k_split_waves_split_along_k(ctx, pool, m, n, k, ta, tb, tc, splits):
 @pytest.mark.parametrize("m,n,k,ta,tb,tc,splits", [(1024, 1024, 16384, False, True, False, 8),
                                                    (1024, 2048, 8192, True, False, True, 4)])
 def test_pipelined_kernel_split_along_k(ctx, pool, m, n, k, ta, tb, tc, splits):
-    """Split-K on the pipelined 128x128 kernel (outputs too large for the 64x64 K-split
+    """Split-K on the pipelined plan's 128x128 tiles, run by the three-piece kernel (outputs too large for the 64x64 K-split
     waves): raw partials in chunks of 2048, added in split order by the reduction; (K, K) and,
     with C column-major, the swapped product; against crates/cpu on every element, the same
     bits over two runs."""
@@ -955,6 +961,7 @@ def test_pipelined_kernel_split_along_k(ctx, pool, m, n, k, ta, tb, tc, splits):
     Cc.upload()
     C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
     assert np.array_equal(first.view(np.uint32), Cc.read().view(np.uint32))
+    assert [x for x in ctx.launches() if x.startswith("gemm")][-1].startswith("gemm_f32_b3<")
     _gemm_fast_check(f"pipelined split {m}x{n}x{k} ta={ta} tb={tb} tc={tc}", first, A.host, la,
                      B.host, lb, c0, lc, m, n, k, alpha, beta)
 
@@ -985,6 +992,7 @@ def test_pipelined_128x64_tiles(ctx, pool, m, n, k, ta, tb, tc):
     Cc.upload()
     C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
     assert np.array_equal(first.view(np.uint32), Cc.read().view(np.uint32))
+    assert [x for x in ctx.launches() if x.startswith("gemm")][-1].startswith("gemm_f32_pl_n64<")
     _gemm_fast_check(f"pipelined 128x64 {m}x{n}x{k} ta={ta} tb={tb} tc={tc}", first, A.host, la,
                      B.host, lb, c0, lc, m, n, k, alpha, beta)
 
@@ -997,13 +1005,13 @@ def test_pipelined_128x64_tiles(ctx, pool, m, n, k, ta, tb, tc):
                                                    (2048, 2048, 2048, False, False, False, 128),
                                                    (2048, 2048, 1152, True, True, True, 128)])
 def test_pipelined_kernel(ctx, pool, m, n, k, ta, tb, tc, tile_m):
-    """Full tiles on the software-pipelined kernel. Grids of 512 128x128 tiles (16-deep
-    slices): every operand layout ((K, MN), (MN, MN), (MN, K) and, with C column-major, the
+    """Full tiles of the software-pipelined plans, run by the three-piece kernels on the same tiles (the pipelined
+    kernels themselves: test_wide_pitch_gpu.py). Grids of 512 128x128 tiles: every operand layout ((K, MN), (MN, MN), (MN, K) and, with C column-major, the
     swapped product), alpha != 1 (fragments scaled as they are read) with beta != 0, K of one
     pipeline step (64) and of several; those whose A-role operand is contiguous along K run as
-    256 tiles of 256x128 with eight waves (gemm_f32_pl256). (K, K) operands with K >= 4096
-    (32-deep slices, K = 4224: 132 slices). Grids of 256 tiles (one workgroup per compute
-    unit, 32-deep slices), also swapped. Against crates/cpu on every element; the same bits
+    256 tiles of 256x128 with eight waves. (K, K) operands with K >= 4096
+    (K = 4224). Grids of 256 tiles (one workgroup per compute
+    unit), also swapped. Against crates/cpu on every element; the same bits
     over two runs."""
     pick = lambda t, r, c: Layout.transposed(r, c) if t else Layout.dense([r, c])
     la, lb, lc = pick(ta, m, k), pick(tb, k, n), pick(tc, m, n)
@@ -1021,6 +1029,7 @@ def test_pipelined_kernel(ctx, pool, m, n, k, ta, tb, tc, tile_m):
     Cc.upload()
     C.gemm(ctx, alpha, A.view(), B.view(), beta, Cc.view())
     assert np.array_equal(first.view(np.uint32), Cc.read().view(np.uint32))
+    assert [x for x in ctx.launches() if x.startswith("gemm")][-1].startswith("gemm_f32_b3")
     _gemm_fast_check(f"pipelined {m}x{n}x{k} ta={ta} tb={tb} tc={tc}", first, A.host, la,
                      B.host, lb, c0, lc, m, n, k, alpha, beta)
 
@@ -1033,9 +1042,8 @@ def test_pipelined_kernel(ctx, pool, m, n, k, ta, tb, tc, tile_m):
                                                   (4096, 4096, 1088, False, 1, False, True),
                                                   (1024, 1024, 256, False, 16, False, True)])
 def test_pipelined_256x256_tiles(ctx, pool, m, n, k, tc, batch, bk, ab):
-    """A row-major with B transposed (K, K) or row-major (K, MN, whose B loads go out apart from
-    the A loads), 256x256 tiles numbering at least one per compute unit: gemm_f32_pl2x (eight
-    waves of 4x2 blocks). 256 tiles; with C column-major (the swapped product, K = 1088: 17
+    """A row-major with B transposed (K, K) or row-major (K, MN), 256x256 tiles numbering at least one per
+    compute unit: gemm_f32_b3_256x256 (eight waves of 4x2 blocks). 256 tiles; with C column-major (the swapped product, K = 1088: 17
     pipeline steps); 16 batches of 16 tiles; K = 4160 (65 steps), which 128x128 tiles would take
     on 32-deep slices; alpha != 1 with beta != 0 where marked, else C filled with NaN (beta = 0
     never reads it). Against crates/cpu on every element of every batch; the same bits over

@@ -1,4 +1,5 @@
-"""Stream-K GEMM (gemm_f32_sk) parity on the GPU.
+"""Stream-K GEMM parity on the GPU: gemm_f32_b3sk, on the runs, slots and tickets of gemm_f32_sk (which wide pitches
+keep, test_wide_pitch_gpu.py).
 
 Products of full 128x128 tiles that a plain grid would spread unevenly over the 256 compute
 units (the busiest one holding more than 10/9 of the mean) run as 256 equal runs of pipeline
@@ -66,6 +67,7 @@ def _run(ctx, pool, m, n, k, seed, a_t=False, b_t=False, c_t=False, batch=1, alp
             Cb.write(c0)
         C.gemm(ctx, alpha, av, bv, beta, cv)
         outs.append(Cb.read(np.float32, count=batch * m * n).copy())
+    assert ctx.launches()[-1].startswith("gemm_f32_b3sk<")
     for o in outs[1:]:
         assert np.array_equal(o.view(np.uint32), outs[0].view(np.uint32)), "not deterministic"
     return a, b, c0, outs[0]
