@@ -77,18 +77,20 @@ def test_tile_edges(ctx, pool, m, n, k, ta, tb, stride, alpha, beta):
     _check(got, a, b, alpha, beta, c0)
 
 
-def test_pieces_hold_the_element_whole(ctx, pool):
-    """A times a permutation matrix is A's columns, bit for bit, over f32's range down to 2^-100."""
+@pytest.mark.parametrize("dense", ["a", "b"])
+def test_pieces_hold_the_element_whole(ctx, pool, dense):
+    """A times a permutation matrix is A's columns, bit for bit, and a permutation matrix times B is B's rows, from f32's
+    least subnormals to 2^103."""
     n = 2048
     g = rng(9200)
-    a = np.ldexp(g.uniform(1, 2, (n, n)), g.integers(-100, 100, (n, n))).astype(np.float32)
-    a *= g.choice([-1, 1], (n, n)).astype(np.float32)
+    x = np.ldexp(g.uniform(1, 2, (n, n)), g.integers(-149, 103, (n, n))).astype(np.float32)
+    x *= g.choice([-1, 1], (n, n)).astype(np.float32)
     perm = g.permutation(n)
-    b = np.zeros((n, n), np.float32)
-    b[perm, np.arange(n)] = 1.0
-    got, name = _product(ctx, pool, a, b, False, False)
+    one = np.zeros((n, n), np.float32)
+    one[perm, np.arange(n)] = 1.0
+    got, name = _product(ctx, pool, *((x, one) if dense == "a" else (one.T.copy(), x)), False, False)
     assert name.startswith("gemm_f32_b3"), name
-    assert np.array_equal(got, a[:, perm])
+    assert np.array_equal(got, x[:, perm] if dense == "a" else x[perm])
 
 
 @pytest.mark.parametrize("shape", [(2045, 1930, 77), (1000, 1020, 1537), (2304, 2304, 256)])
@@ -214,3 +216,31 @@ def test_long_sums_are_not_biased(ctx, pool, m, n, k, kernel, what):
     # The mean over 64 n outputs of errors that are independent of each other strays by 2e-8 of the magnitude at
     # the most (an rms error of 1.4 1.8e-8 sqrt(K), over sqrt(64 n)); a turn's own share is 5e-8.
     assert abs(err.mean()) <= 1.2e-7 * np.abs(want).mean(), err.mean() / np.abs(want).mean()
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_single_products(ctx, pool, kernel):
+    """Rows of one element each, so that every output is one product of two full mantissas: the six products of pieces
+    that are formed leave out 2^-24 of it at the most, the last addition cuts up to 2^-23 (or rounds), and
+    the five before it are below 2^-7 of it and err by 2^-28 in all. Without any one of the six the worst output is 2^-17 off or more."""
+    m, n, k, ta = KERNELS[kernel]
+    g = rng(9900 + m)
+    a, b = np.zeros((m, k), np.float32), g.uniform(1, 2, (k, n)).astype(np.float32)
+    a[np.arange(m), np.arange(m) % k] = g.uniform(-2, 2, m)
+    got, name = _product(ctx, pool, a, b, ta, False)
+    assert name.startswith(kernel), name
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.max(np.abs(got - want) / np.abs(want)) <= 1.6 * 2.0 ** -23
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_error_in_norm(ctx, pool, kernel):
+    """Normal operands: the error's norm over the result's is an f32 chain's, 1.8e-8 sqrt(K), or less (measured: 1.1e-7 at
+    K = 64, 3.5e-7 at 1537). Any five of the six products would leave 2.4e-6 or more at K = 64."""
+    m, n, k, ta = KERNELS[kernel]
+    g = rng(9950 + m)
+    a, b = g.standard_normal((m, k)).astype(np.float32), g.standard_normal((k, n)).astype(np.float32)
+    got, name = _product(ctx, pool, a, b, ta, False)
+    assert name.startswith(kernel), name
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.linalg.norm(got - want) <= 1.8e-8 * np.sqrt(k) * np.linalg.norm(want)
