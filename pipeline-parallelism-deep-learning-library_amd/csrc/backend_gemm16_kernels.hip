@@ -224,7 +224,7 @@ __global__ __launch_bounds__(QT) void gemm16_seq(Gemm16SeqArgs p) {
 // ones can, so a slice that holds an |alpha * a| or |b| outside [2^-55, 2^62) that is not zero takes separate
 // multiplies and adds from the same stage (multiply_odd), at the VALU's rate: softmax weights and small gradients
 // are there as a matter of course. us, one such element / some in every slice / gemm16_seq: 2048 x 4096 x 1024
-// 162 / 365 / 420 (165 without any), 1501 x 1477 x 1023 75 / 171 / 174 (73), 128 x 1408 x 1024 17 / 51 / 128 (14.6); with
+// 158 / 362 / 420 (160 without any), 1501 x 1477 x 1023 73 / 171 / 174 (70), 128 x 1408 x 1024 17 / 51 / 128 (14.2); with
 // whole tiles computed again from memory 763 / 642, 354 / 360 and 185 / 186.
 // A last slice that is not full is padded with products (-0) * 1: adding -0 changes no sum.
 //
@@ -334,16 +334,22 @@ __global__ __launch_bounds__(256, 2) void gemm16_chain(Gemm16SeqArgs p) {
                 f[j] = scale * widen<HK>(h);
             }
             if constexpr (HK == 1) {
-                // Two instructions an element: twice the magnitude's bits less one (zero: the largest), and the
-                // least of three; the largest magnitude of three, in which NaNs do not count (nor need they).
-                uint32_t low = 0xffffffffu;
-                float high = 0.0f;
+                // One instruction an element for the least and the largest magnitude (NaNs do not count, nor need
+                // they); where zeros or small elements are among them, the least that is not zero: twice its bits less
+                // one, which makes zero the largest. (Four instructions an element for all: 4096^3 1185 -> 1162 us.)
+                constexpr float LEAST = 0x1p-55f, LARGEST = 0x1p62f;
+                float least = LARGEST, most = 0.0f;
 #pragma unroll
                 for (int j = 0; j < 16; j += 2) {
-                    low = min(low, min((__builtin_bit_cast(uint32_t, f[j]) << 1) - 1, (__builtin_bit_cast(uint32_t, f[j + 1]) << 1) - 1));
-                    __asm__("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(high) : "v"(f[j]), "v"(f[j + 1]));
+                    __asm__("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(least) : "v"(f[j]), "v"(f[j + 1]));
+                    __asm__("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(f[j]), "v"(f[j + 1]));
                 }
-                if (__any(low < ((127u - 55u) << 24) - 1 || high >= 0x1p62f)) odd_slice[s & 1] = s + 1;
+                if (__any(least < LEAST || most >= LARGEST)) {
+                    uint32_t low = 0xffffffffu;
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) low = min(low, (__builtin_bit_cast(uint32_t, f[j]) << 1) - 1);
+                    if (__any(low < (__builtin_bit_cast(uint32_t, LEAST) << 1) - 1 || most >= LARGEST)) odd_slice[s & 1] = s + 1;
+                }
             }
             if (k + 16 > p.k) {
 #pragma unroll
