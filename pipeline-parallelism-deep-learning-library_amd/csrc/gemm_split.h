@@ -3,9 +3,11 @@
 // An f32 has 24 significant bits and a bf16 has 8, so x = x0 + x1 + x2 with x0 = bf16(x),
 // x1 = bf16(x - x0), x2 = x - x0 - x1, each step exact: the three pieces hold the f32 whole. A
 // product is then six bf16 products, a0b0 + (a0b1 + a1b0) + (a1b1 + a0b2 + a2b0); the three left
-// out are below 2^-26 of it. bf16 products are exact in f32 and one
+// out add up to 2^-24 of it at the most. bf16 products are exact in f32 and one
 // v_mfma_f32_32x32x16_bf16 adds sixteen of them into an f32 accumulator, so a sum over K is
-// rounded about 6 K / 16 times instead of the K times of v_mfma_f32_32x32x2_f32.
+// rounded about 6 K / 16 times instead of the K times of v_mfma_f32_32x32x2_f32. A sum of many terms is closer to
+// the exact one for it; one of a single term, which that instruction rounds correctly, is up to 1.5 units in
+// the last place off (measured: 1.48, one in five not the nearest f32).
 //
 // Elements are scaled by 2^23 before they are split and the sums by 2^-46 after: an f32, subnormals
 // included, is a whole multiple of 2^-149, so a scaled one is a whole multiple of 2^-126 and each of its pieces
@@ -531,8 +533,9 @@ __device__ __forceinline__ uint32_t b3_sums(const GemmArgs& p, char* smem, const
 // they are split, so a load needs no alignment beyond its elements' and edges cost no second path.
 //
 // Bound: the chip's power. 1748 TFLOP/s of bf16 MFMA is what it sustains with nothing else running (1.74 of
-// 2.4 GHz), 291 TFLOP/s of this product; the 256x256 tiles keep the matrix cores 78 % busy at 1.70 GHz, the
-// rest of the power going into fragment reads and conversions. Fewer stalls alone do not help: the same
+// 2.4 GHz), 291 TFLOP/s of this product; the 256x256 tiles keep the matrix cores 79 % busy at 1.6-1.7 GHz (4096^3), the
+// rest of the power going into fragment reads and conversions. 128x128 tiles are 48 % busy at 2.07 GHz on one workgroup per
+// compute unit (2048^3), 62 % at 1.83 on many (2048 x 8192 x 2048): their two waves per SIMD or fewer wait. Fewer stalls alone do not help: the same
 // kernel without a schedule was busy 69 % at 1.87 GHz and 3 % slower. Against v_mfma_f32_32x32x2_f32 on the same
 // tiles: 4096^3 931 -> 570-580 us (148 -> 237 TFLOP/s), 32 x 1024^3 483 -> 310 us (142 -> 222), a layer's three
 // products and elementwise work at 2048 x 2048 x 8192 1554 -> 1108 us. Error against f64 on
@@ -593,10 +596,10 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
 // of 32x32 sharing stages would read twice that, the LDS's whole rate), and nothing but its own loads
 // and LDS accesses, which complete in order, holds it: no barrier before the end, one stage a wave. The price is the
 // conversion, once per wave: 208 VALU instructions for 24 MFMAs, more than they hide, so two workgroups
-// share a compute unit. The sums meet in LDS as (s0 + s1) + (s2 + s3), each wave storing one block. Bound:
-// the VALU, at 110-115 TFLOP/s. Against the f32 instruction: 3001 x 2011 x 1537 with odd rows 459 -> 164 us
-// (32-bit loads before), 2300 x 2304 x 2304 274 -> 219, 320 x 352 x 97536 418 -> 224, 37^6 in rank 4 147 -> 56,
-// 1000 x 1024 x 1024 with A along M 40 -> 30.
+// share a compute unit. The sums meet in LDS as (s0 + s1) + (s2 + s3), each wave storing one block. Bound: what a wave
+// waits for, at 110-118 TFLOP/s: matrix cores 28 % busy, VALU 38 %, LDS 22 % (2300 x 2304 x 2304, 2.1 GHz). Against the f32 instruction: 3001 x 2011 x 1537 with odd rows 459 -> 164 us
+// (32-bit loads before), 2300 x 2304 x 2304 274 -> 214, 320 x 352 x 97536 418 -> 224, 37^6 in rank 4 147 -> 56,
+// 1000 x 1024 x 1024 with A along M 40 -> 27.
 template <int AM, int BMD, bool EDGE>
 __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     constexpr int R = 64, W = 4;
@@ -738,8 +741,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
 
 // gemm_f32_b3sk<AM, BMD, TURNS>: gemm_f32_sk's runs, slots and tickets (gemm_pipe.h) over the three-piece
 // sums of full 128x128 tiles: each run's part of a tile is checked, and summed again where it must be, before
-// it meets the other run's. One workgroup per compute unit. 48^6 in rank 4 (2304^3): 185 -> 149 us, 164 TFLOP/s,
-// with one wave per SIMD; 2048^3, the same wave on whole tiles, 126 -> 98 us.
+// it meets the other run's. One workgroup per compute unit. 48^6 in rank 4 (2304^3): 185 -> 147 us, 166 TFLOP/s,
+// with one wave per SIMD, the matrix cores 47 % busy at 2.0 GHz; 2048^3, the same wave on whole tiles, 126 -> 95 us.
 template <int AM, int BMD, B3Turns TURNS>
 __global__ __launch_bounds__(256, 1) void gemm_f32_b3sk(GemmArgs p) {
     constexpr int FM = 2, FN = 2, RA = 128, RB = 128, SLOT = 128 * 128, STEP = 128;
