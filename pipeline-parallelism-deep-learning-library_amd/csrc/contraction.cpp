@@ -522,13 +522,19 @@ void plan_half(const View& a, const View& b, const View& c, const Merged& mg, fl
     t.beta = beta;
     // The tile kernel wants whole tiles and slices of aligned operands, two workgroups of them per compute unit;
     // everything else whose rows lie within 32 bits of bytes goes to gemm_f16_edge, on 32x32 tiles
-    // where 64x64 ones would be fewer than that and K is at least one slice.
+    // where 64x64 ones would be fewer than that and K is at least one slice. A K of less than a slice takes
+    // the edge kernel's element loads of an operand along M or N, 16 in turn behind predicates, so it stays with
+    // the tile kernel (72 x 1528 x 32: 10.4-10.6 us against 11.7-13.3) unless both operands lie along K (11.1 against
+    // 10.4), or one does on a large grid whose rows are all unaligned (2001 x 1999 x 32: 23.3 against 22.5).
     auto near = [](uint64_t s_row, uint64_t s_k) { return s_row < (1u << 22) && s_k < (1u << 22); };
     const uint64_t big = gemm_half_workgroups(m, n, batch, HGEMM_BM);
     const bool whole = m % HGEMM_BM == 0 && n % HGEMM_BN == 0 && k % HGEMM_BK == 0 &&
                        info.a_mode != LG_LOAD_STRIDED && info.b_mode != LG_LOAD_STRIDED;
     const bool few = big < 2 * GEMM_CUS && k >= HGEMM_BK;
-    t.edge = (!whole || few) && near(am.a, ak.a) && near(an.b, ak.b) ? 1 : 0;
+    const int along_k = (ak.a == 1) + (ak.b == 1);
+    const bool deep = k >= HGEMM_BK || along_k == 2 ||
+                      (along_k == 1 && big >= 2 * GEMM_CUS && info.a_mode == LG_LOAD_STRIDED && info.b_mode == LG_LOAD_STRIDED);
+    t.edge = (!whole || few) && deep && near(am.a, ak.a) && near(an.b, ak.b) ? 1 : 0;
     t.tile = t.edge != 0 && few ? 32 : HGEMM_BM;
     t.tiles_m = (m + t.tile - 1) / t.tile;
     t.tiles_n = (n + t.tile - 1) / t.tile;

@@ -29,8 +29,29 @@ def test_edges_round_once(ctx, pool, m, n, k, at, bt, stride, offset):
     c0 = grid_halves(g, m * n) if beta else np.full(m * n, np.nan, np.float16)
     c = Half(pool, Layout.dense([m, n]), c0)
     C.gemm(ctx, alpha, a.view(), b.view(), beta, c.view())
-    assert ctx.launches()[-1].startswith("gemm_f16_edge") or m % 64 == n % 64 == k % 64 == 0
+    # Less than a slice of K: only operands that both lie along it.
+    edge = k >= 64 or (not at and bt)
+    assert ctx.launches()[-1].startswith("gemm_f16_edge" if edge else "gemm_f16_f64mfma")
     want = alpha * (a.logical().astype(np.float64) @ b.logical().astype(np.float64))
     if beta:
         want = want + beta * c0.reshape(m, n).astype(np.float64)
+    assert f16_bits_equal(c.read()[: m * n].reshape(m, n), want.astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,edge", [(72, 1528, ()), (1000, 1001, ()), (2001, 1999, ((False, False), (True, True))),
+                                      (2000, 2000, ())])
+def test_short_k_keeps_the_tile_kernel(ctx, pool, m, n, edge, at, bt):
+    """K of half a slice: the edge kernel where both operands lie along K, or one on a large grid of unaligned
+    rows; elsewhere its predicated element loads took up to 28 % longer than the tile kernel."""
+    k = 31
+    g = rng(8750 + m)
+    la = Layout(0, [m, k], [1, m] if at else [k, 1])
+    lb = Layout(0, [k, n], [1, k] if bt else [n, 1])
+    a, b = Half(pool, la, grid_halves(g, la.span())), Half(pool, lb, grid_halves(g, lb.span()))
+    c = Half(pool, Layout.dense([m, n]), np.full(m * n, np.nan, np.float16))
+    C.gemm(ctx, 1.0, a.view(), b.view(), 0.0, c.view())
+    along_k = not at and bt
+    assert ctx.launches()[-1] == ("gemm_f16_edge" if along_k or (at, bt) in edge else "gemm_f16_f64mfma")
+    want = a.logical().astype(np.float64) @ b.logical().astype(np.float64)
     assert f16_bits_equal(c.read()[: m * n].reshape(m, n), want.astype(np.float16).view(np.uint16))
