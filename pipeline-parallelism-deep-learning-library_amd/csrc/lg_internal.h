@@ -352,11 +352,11 @@ struct PermTileArgs {
     int64_t src_sb, dst_sa;           // source stride of b, destination stride of a
     uint32_t outer_rank;
     uint32_t tiles_a, tiles_b;
+    uint32_t order;  // walk over the tiles, set at the launch (perm_tile_order)
     uint64_t total_tiles;
     uint32_t outer_shape[PERM_MAX_RANK];
     int64_t outer_src[PERM_MAX_RANK];
     int64_t outer_dst[PERM_MAX_RANK];
-    uint32_t order;  // walk over the tiles, set at the launch (perm_tile_order)
 };
 
 struct PermCopyArgs {

@@ -193,12 +193,17 @@ uint64_t perm_copy_workgroups(uint64_t count, int words) {
 // cut: rows on the grid (77088 x 229 35.0 against 41.4), one tile per row ([28,1372,240] by 1,2,0 16.7
 // against 18.8), streaming tiles (8192 x 4096 48.6 against 49.5); and on aligned rows of many planes
 // ([100,180,16,36] by 2,0,3,1 22.9 against 24.6; unaligned [66,30,47,8] by 3,1,2,0 gains, 15.6 -> 12.9).
+// Two tiles along a of which the last is at least half full, but not full, also lose (20001 x 112 7.6 by order 0 against 8.1 by
+// order 2, 9922 x 120 5.6 against 6.2, 100001 x 96 18.5 against 20.1; 40003 x 120 alone 13.7 against 13.1); an emptier
+// one gains (100001 x 88 19.2 against 17.4, 40003 x 80 9.2 against 8.5), and so does a full one (100001 x 128 19.5 against 16.9).
 uint32_t perm_tile_order(const PermTileArgs& a, int words, bool vec, bool streaming) {
     constexpr uint32_t FEW = 32;
     if (streaming || a.tiles_b < 2 || (a.dst_sa * words) % 32 == 0 || (vec && a.outer_rank != 0) ||
         a.total_tiles > 0xffffffffull) {
         return 0;
     }
+    const uint32_t last = a.ext_a % PERM_TILE_A;
+    if (a.outer_rank == 0 && a.tiles_a == 2 && last >= PERM_TILE_A / 2) return 0;
     return a.outer_rank == 0 && a.tiles_b > a.tiles_a && a.tiles_a <= FEW ? 2 : 1;
 }
 

@@ -14,6 +14,9 @@ pytestmark = pytest.mark.gpu
     ([2081, 2053], [1, 0]),      # runs, b first: 33 x 33 tiles
     ([70, 66], [1, 0]),          # four tiles for eight XCDs
     ([5, 3, 65, 67], [0, 1, 3, 2]),  # runs over planes
+    ([1301, 95], [1, 0]),        # runs, a first, the second tile less than half full
+    ([1301, 96], [1, 0]),        # half full and one short of full: plain
+    ([1301, 127], [1, 0]),
     ([6, 132, 36], [0, 2, 1]),   # aligned planes: plain
     ([96, 200], [1, 0]),         # destination rows on the 128-byte grid: plain
 ])
