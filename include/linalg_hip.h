@@ -459,7 +459,8 @@ typedef struct lg_contract_plan {
                              (2 for 128x128 tiles, 4 for 64x64); LG_KERNEL_PIPELINED on 64x64
                              tiles: 4 (each wave takes a quarter of every K chunk); else 1 */
     uint32_t reserved;
-    /* f32 plans of 64x64 tiles and more (but 128x64) with K chunks of 64 and more (64x64: 256 or 512), row
+    /* f32 plans of 64x64 tiles and more (but 128x64) with K chunks of 64 and more (64x64: 256 or 512; whole K
+     * with a part of 16 left along both operands' unit strides 80, short sums into outputs of 128 MB and 128 or 256 rows 96 or 160), row
      * pitches below 2^20 and K strides below 2^23 elements keep their tiles, grid and splits but multiply on the bf16 matrix cores, every element as three bf16 pieces that
      * hold it whole (csrc/gemm_split.h); the launch log names the kernel gemm_f32_b3*. There a
      * 64x64 tile has kgroups 4, and a 128x128 one one wave group whatever kgroups says. */

@@ -427,13 +427,27 @@ int load_mode_half(uintptr_t base, uint64_t off, uint64_t sb, uint64_t srow, uin
 // against 31 (17 x 880 x 176), 1008 deep 90 against 81 (12 x 896 x 368); and whole K over four
 // wave groups with A along K 28.8 against 29.5 (1024 x 1024 x 1000), A along M 40 against 30. Full 64x64 tiles on
 // gemm_f32_kw gain too little to move (256 x 256 x 65536 77.0 against 75.7).
+// Aligned operands gain from 64 k on (1.0-1.35 times the f32 kernels' rate at K = 64-120), with two exceptions. A
+// tail of less than a slice along K is fetched with 32-bit loads, by both operands where both are contiguous there:
+// 2048 x 2048 x 72 0.94, 128 x 32768 x 72 0.94, 0.98-1.05 at 88. And one or two rows of tiles whose output
+// goes past half the Infinity Cache are bound by its stores, which one workgroup per compute unit overlaps
+// less well: 256 of 128 x 1024 0.93-0.99 at K = 64-80, 1.0 from 96 (of both along K with a tail 0.96 at 136, 0.99 at
+// 152); half the output gains, 128 of 128 x 1024 1.03-1.15, and so do 256x256 tiles (256 x 262144 x 64 1.28),
+// partly filled ones (600 of 120 x 512 1.1-1.2) and three rows (200 of 384 x 640 x 80 1.08). Other operands take 32-bit
+// loads on the f32 kernels too, and gain at every K.
 bool pieces_fit(const GemmArgs& t, int a_mode, int b_mode) {
     if (t.kernel != KERN_TILE && t.kernel != KERN_DIRECT && t.kernel != KERN_PIPE && t.kernel != KERN_SK) return false;
     if (t.tile < GEMM_SMALL_TILE || (t.tile != PIPE_TALL_M && t.tile_n < t.tile)) return false;
     const uint32_t last = t.k - (t.splits - 1) * t.k_chunk;
     if (std::min(t.k_chunk, last) < PIECES_MIN_K || t.m < 4 || t.n < 4) return false;
+    const bool aligned = a_mode != LOAD_S && b_mode != LOAD_S;
+    if (aligned && t.splits == 1) {
+        const bool tail = last % 16 != 0 && a_mode == LOAD_K && b_mode == LOAD_K;
+        const bool streams = t.m <= 2 * GEMM_BM && t.m % GEMM_BM == 0 && t.tile != PIPE_TALL_M &&
+                             static_cast<uint64_t>(t.m) * t.n * t.batch >= PIECES_STREAM;
+        if (last < (streams ? (tail ? 160u : 96u) : tail ? 80u : PIECES_MIN_K)) return false;
+    }
     if (t.tile == GEMM_SMALL_TILE) {
-        const bool aligned = a_mode != LOAD_S && b_mode != LOAD_S;
         if (t.k_chunk < (aligned ? 512u : 256u)) return false;
         if (t.kernel == KERN_PIPE || (t.kernel == KERN_DIRECT && a_mode == LOAD_K)) return false;
     }

@@ -199,6 +199,8 @@ struct GemmArgs {
 static_assert(sizeof(GemmArgs) + sizeof(uint32_t) <= 3 * 64, "GemmArgs and the grid's size fill three lines");
 // K chunks below this stay on the f32 matrix instruction.
 constexpr uint32_t PIECES_MIN_K = 64;
+// Elements of an output past half the Infinity Cache (128 MB): short sums into it are bound by its stores.
+constexpr uint64_t PIECES_STREAM = 1ull << 25;
 // Launches the three-piece kernel for args.pieces; returns the name for the launch log.
 const char* launch_gemm_pieces(hipStream_t s, const GemmArgs& args, uint32_t groups);
 

@@ -77,6 +77,32 @@ def test_tile_edges(ctx, pool, m, n, k, ta, tb, stride, alpha, beta):
     _check(got, a, b, alpha, beta, c0)
 
 
+@pytest.mark.parametrize("m,n,k,ta,tb,kernel", [
+    (2048, 2048, 72, False, True, "gemm_f32_dl"),     # both along K, a tail of 8
+    (2048, 2048, 84, False, True, "gemm_f32_b3<"),    # tails of 4, 8 and 12
+    (2048, 2048, 88, False, True, "gemm_f32_b3<"),
+    (2048, 2048, 92, False, True, "gemm_f32_b3<"),
+    (2048, 2048, 72, False, False, "gemm_f32_b3<"),   # A along K alone
+    (4096, 4096, 65, True, False, "gemm_f32_b3"),     # neither along K: tails of 1 and 15
+    (4096, 4096, 79, True, False, "gemm_f32_b3"),
+    (128, 262144, 64, False, False, "gemm_f32_pl"),   # one row of tiles, an output of 128 MB
+    (128, 262144, 88, False, False, "gemm_f32_dl"),
+    (128, 262144, 96, False, False, "gemm_f32_b3"),
+    (128, 262144, 136, False, True, "gemm_f32_dl"),
+    (256, 131072, 64, False, False, "gemm_f32_b3_256x256"),
+    (128, 131072, 64, False, False, "gemm_f32_b3<"),  # and of 64 MB
+])
+def test_short_sums(ctx, pool, m, n, k, ta, tb, kernel):
+    """Sums of a few slices on the kernel that is the faster one for them, their last slice partly filled."""
+    g = rng(9300 + m + n + k)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+    got, name = _product(ctx, pool, a, b, ta, tb)
+    assert name.startswith(kernel), name
+    columns = slice(n % 7, None, max(1, n // 4099))
+    _check(got[:, columns], a, b[:, columns], 1.0, 0.0, None)
+
+
 @pytest.mark.parametrize("dense", ["a", "b"])
 def test_pieces_hold_the_element_whole(ctx, pool, dense):
     """A times a permutation matrix is A's columns, bit for bit, and a permutation matrix times B is B's rows, from f32's
