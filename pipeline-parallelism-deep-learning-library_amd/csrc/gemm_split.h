@@ -602,9 +602,9 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN >= 8 ? 1 : 2) void gemm_f32_b
 // and LDS accesses, which complete in order, holds it: no barrier before the end, one stage a wave. The price is the
 // conversion, once per wave: 208 VALU instructions for 24 MFMAs, more than they hide, so two workgroups
 // share a compute unit. The sums meet in LDS as (s0 + s1) + (s2 + s3), each wave storing one block. Bound: what a wave
-// waits for, at 110-118 TFLOP/s: matrix cores 28 % busy, VALU 38 %, LDS 22 % (2300 x 2304 x 2304, 2.1 GHz). Against the f32 instruction: 3001 x 2011 x 1537 with odd rows 459 -> 164 us
-// (32-bit loads before), 2300 x 2304 x 2304 274 -> 214, 320 x 352 x 97536 418 -> 224, 37^6 in rank 4 147 -> 56,
-// 1000 x 1024 x 1024 with A along M 40 -> 27.
+// waits for, at 110-118 TFLOP/s: matrix cores 28 % busy, VALU 38 %, LDS 22 % (2300 x 2304 x 2304, 2.1 GHz). Against the
+// f32 instruction: 1000 x 1020 x 1537 with odd rows 148-162 -> 29-34 us (32-bit loads before), 2300 x 2304 x 2304 274 -> 214,
+// 320 x 352 x 97536 418 -> 224, 37^6 in rank 4 147 -> 56, 1000 x 1024 x 1024 with A along M 40 -> 27.
 template <int AM, int BMD, bool EDGE>
 __global__ __launch_bounds__(256, 2) void gemm_f32_b3kw(GemmArgs p) {
     constexpr int R = 64, W = 4;
